@@ -394,20 +394,20 @@ WPT_HD bool querySphere(const DevScene& s, const Ray& ray, uint32_t index, bool 
 // query -- run the same node-visit code in the same iteration.
 //
 // TlasWalk is the same query as a resumable walk: start() runs the
-// categories before the TLAS and enters its root, step() makes one
-// iteration of traceQuery's loop (one node or leaf), finish() runs the
-// categories after the TLAS.  A kernel can thus interleave the walks of
-// several rays in one lane (a lane whose ray ends starts its next one while
-// the other lanes of its wave still walk theirs); each ray's visits, and so
-// its result, are those of traceQuery.  traceQuery keeps its own loop: as
-// start/step/finish its code is slower (the sphere field's closest-hit pass: 69 -> 80 ms
-// per 64-sample frame).
+// categories before the TLAS and enters its root, visitNode() and visitLeaf()
+// each make one iteration of traceQuery's loop, finish() runs the categories
+// after the TLAS.  A kernel can thus interleave the walks of several rays in
+// one lane, and choose for a whole wave which kind of visit runs next; each
+// ray's visits, and so its result, are those of traceQuery.  traceQuery keeps
+// its own loop: as start/visit/finish its code is slower (the sphere field's
+// closest-hit pass: 69 -> 80 ms per 64-sample frame).
 enum class Walk { kTlas, kAfter, kDone };  // walking the TLAS; categories after it left; complete
 
 template <bool Full, Query Q>
 struct TlasWalk {
     Ray ray;
     RayInv r;
+    Vec3 worldInv;  // 1 / ray.direction
     HitRecord best;
     const BvhNode* nodes;
     const float4* geometry;
@@ -437,6 +437,7 @@ struct TlasWalk {
             return Walk::kDone;
         if (s.tlas.primCount == 0) return Walk::kAfter;
         r = makeRayInv(ray);
+        worldInv = r.inv;
         float nearT;
         if (!slab(r, s.tlas.rootMin[0], s.tlas.rootMin[1], s.tlas.rootMin[2], s.tlas.rootMax[0], s.tlas.rootMax[1],
                 s.tlas.rootMax[2], best.t, nearT))
@@ -451,86 +452,97 @@ struct TlasWalk {
         return Walk::kTlas;
     }
 
+    // The next live entry of the level being walked; when a BLAS is
+    // exhausted, of the TLAS around it.
     template <class Stack>
-    WPT_HD Walk step(const DevScene& s, Stack& stack) {
-        if (cur & kLeafBit) {
-            uint32_t slot = cur & ~kLeafBit;
-            if (instance != kInvalid) {
-                float4 a = geometry[3 * slot + 0];
-                float4 b = geometry[3 * slot + 1];
-                float4 c = geometry[3 * slot + 2];
-                float t, u, v;
-                if (intersectTriangle(r.ray, xyz(a), xyz(b), xyz(c), t, u, v) &&
-                    wanted(any(), t, kRankTlasInstance, instance, wbits(a), best)) {
-                    uint32_t material = materialOverride == kInvalid ? wbits(b) : materialOverride;
-                    if (s.materialCutout[material] == kCutNever ||
-                        !cutAway<Full>(s, material, s.blases[s.instances[instance].mesh].triangles, wbits(a), u, v)) {
-                        record(best, t, u, v, kHitInstance, instance, wbits(a), material, kRankTlasInstance);
-                        if (any()) {
-                            stack.truncate(base);
-                            return Walk::kDone;
-                        }
-                    }
-                }
-            } else {
-                uint32_t leaf = s.tlasLeaves[slot];
-                if (leaf & kTlasSphereBit) {
-                    if (querySphere(s, ray, leaf & ~kTlasSphereBit, any(), best)) {
-                        stack.truncate(base);
-                        return Walk::kDone;
-                    }
-                } else {
-                    const Instance& inst = s.instances[leaf];
-                    const Blas& blas = s.blases[inst.mesh];
-                    Ray local = toLocal(inst.transform, ray);
-                    if (blas.bvh.primCount != 0) {
-                        RayInv rl = makeRayInv(local);
-                        float nearT;
-                        if (slab(rl, blas.bvh.rootMin[0], blas.bvh.rootMin[1], blas.bvh.rootMin[2], blas.bvh.rootMax[0],
-                                blas.bvh.rootMax[1], blas.bvh.rootMax[2], best.t, nearT)) {
-                            r = rl;
-                            instance = leaf;
-                            nodes = blas.bvh.nodes;
-                            geometry = blas.geometry;
-                            materialOverride = inst.materialOverride;
-                            blasBase = stack.size;
-                            cur = blas.bvh.root;
-                            return Walk::kTlas;
-                        }
-                    } else if (queryBrute<Full>(s, local, blas.triangles, blas.triangleCount, inst.materialOverride,
-                                   kHitInstance, kRankTlasInstance, leaf, any(), best)) {
-                        stack.truncate(base);
-                        return Walk::kDone;
-                    }
-                }
-            }
-        } else {
-            const BvhNode& n = nodes[cur];
-            float tl, tr;
-            bool hl = slab(r, n.lminx, n.lminy, n.lminz, n.lmaxx, n.lmaxy, n.lmaxz, best.t, tl);
-            bool hr = slab(r, n.rminx, n.rminy, n.rminz, n.rmaxx, n.rmaxy, n.rmaxz, best.t, tr);
-            if (hl && hr) {
-                bool leftNear = tl < tr;
-                stack.push(leftNear ? n.right : n.left, leftNear ? tr : tl);
-                cur = leftNear ? n.left : n.right;
-                return Walk::kTlas;
-            }
-            if (hl) {
-                cur = n.left;
-                return Walk::kTlas;
-            }
-            if (hr) {
-                cur = n.right;
-                return Walk::kTlas;
-            }
-        }
+    WPT_HD Walk next(const DevScene& s, Stack& stack) {
         if (instance != kInvalid) {
             if (popLive(stack, blasBase, best.t, cur)) return Walk::kTlas;
             instance = kInvalid;
             nodes = s.tlas.nodes;
-            r = makeRayInv(ray);
+            r.ray = ray;
+            r.inv = worldInv;
         }
         return popLive(stack, base, best.t, cur) ? Walk::kTlas : Walk::kAfter;
+    }
+
+    WPT_HD bool atLeaf() const { return (cur & kLeafBit) != 0u; }
+
+    // One interior node (atLeaf() is false).
+    template <class Stack>
+    WPT_HD Walk visitNode(const DevScene& s, Stack& stack) {
+        const BvhNode& n = nodes[cur];
+        float tl, tr;
+        bool hl = slab(r, n.lminx, n.lminy, n.lminz, n.lmaxx, n.lmaxy, n.lmaxz, best.t, tl);
+        bool hr = slab(r, n.rminx, n.rminy, n.rminz, n.rmaxx, n.rmaxy, n.rmaxz, best.t, tr);
+        if (hl && hr) {
+            bool leftNear = tl < tr;
+            stack.push(leftNear ? n.right : n.left, leftNear ? tr : tl);
+            cur = leftNear ? n.left : n.right;
+            return Walk::kTlas;
+        }
+        if (hl || hr) {
+            cur = hl ? n.left : n.right;
+            return Walk::kTlas;
+        }
+        return next(s, stack);
+    }
+
+    // One leaf (atLeaf() is true): a BLAS triangle, or a TLAS sphere or
+    // instance, whose BLAS the walk enters.
+    template <class Stack>
+    WPT_HD Walk visitLeaf(const DevScene& s, Stack& stack) {
+        uint32_t slot = cur & ~kLeafBit;
+        if (instance != kInvalid) {
+            float4 a = geometry[3 * slot + 0];
+            float4 b = geometry[3 * slot + 1];
+            float4 c = geometry[3 * slot + 2];
+            float t, u, v;
+            if (intersectTriangle(r.ray, xyz(a), xyz(b), xyz(c), t, u, v) &&
+                wanted(any(), t, kRankTlasInstance, instance, wbits(a), best)) {
+                uint32_t material = materialOverride == kInvalid ? wbits(b) : materialOverride;
+                if (s.materialCutout[material] == kCutNever ||
+                    !cutAway<Full>(s, material, s.blases[s.instances[instance].mesh].triangles, wbits(a), u, v)) {
+                    record(best, t, u, v, kHitInstance, instance, wbits(a), material, kRankTlasInstance);
+                    if (any()) {
+                        stack.truncate(base);
+                        return Walk::kDone;
+                    }
+                }
+            }
+            return next(s, stack);
+        }
+        uint32_t leaf = s.tlasLeaves[slot];
+        if (leaf & kTlasSphereBit) {
+            if (querySphere(s, ray, leaf & ~kTlasSphereBit, any(), best)) {
+                stack.truncate(base);
+                return Walk::kDone;
+            }
+            return next(s, stack);
+        }
+        const Instance& inst = s.instances[leaf];
+        const Blas& blas = s.blases[inst.mesh];
+        Ray local = toLocal(inst.transform, ray);
+        if (blas.bvh.primCount != 0) {
+            RayInv rl = makeRayInv(local);
+            float nearT;
+            if (slab(rl, blas.bvh.rootMin[0], blas.bvh.rootMin[1], blas.bvh.rootMin[2], blas.bvh.rootMax[0],
+                    blas.bvh.rootMax[1], blas.bvh.rootMax[2], best.t, nearT)) {
+                r = rl;
+                instance = leaf;
+                nodes = blas.bvh.nodes;
+                geometry = blas.geometry;
+                materialOverride = inst.materialOverride;
+                blasBase = stack.size;
+                cur = blas.bvh.root;
+                return Walk::kTlas;
+            }
+        } else if (queryBrute<Full>(s, local, blas.triangles, blas.triangleCount, inst.materialOverride, kHitInstance,
+                       kRankTlasInstance, leaf, any(), best)) {
+            stack.truncate(base);
+            return Walk::kDone;
+        }
+        return next(s, stack);
     }
 
     template <class Stack>

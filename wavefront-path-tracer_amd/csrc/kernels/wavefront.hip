@@ -291,13 +291,95 @@ __global__ void kReset(LaunchContext ctx, uint32_t nextSel) {
     }
 }
 
-// Lanes of a wave that wait before they start new rays together (1: each
-// starts its next ray as soon as the last one ends; 64: the wave's rays
-// start and end together).
-#ifndef WPT_TRACE_REFILL
-#define WPT_TRACE_REFILL 16
-#endif
-constexpr int kTraceRefill = WPT_TRACE_REFILL;
+// Lanes of a wave that wait before they start new rays together (16 and 32
+// within 1% of each other on the sphere field and the terrain, 8 slower).
+constexpr int kTraceRefill = 32;
+// A leaf visit is run once the lanes at leaves, counted this many times,
+// outnumber the lanes at nodes (sphere field / terrain, ms of kTrace per 64 /
+// 16 samples: 1: 60.2 / 66.7, 2: 58.4 / 66.2, 3: 58.4 / 67.2, 1/2: 62.7 / 69.5).
+constexpr int kLeafWeight = 2;
+
+// The walks of a wave's rays, one loop over visits: each turn runs either
+// node visits or leaf visits, whichever most lanes stand at, and lanes whose
+// rays ended wait until kTraceRefill of them (or all that are left) store
+// their results and start their next rays together.  A turn that ran both
+// kinds of visit for the lanes that needed either kept a quarter of the
+// lanes of a VALU instruction active, and VALU issue bounds the walk: with
+// turns of one kind the closest-hit passes went from 66.1 to 58.4 ms per
+// 64-sample sphere-field frame (1920x1080) and from 77.5 to 66.2 ms per
+// 16-sample terrain frame, the terrain's event rays from 74.2 to 62.8 ms.  A
+// ray's own visits, and so its result, are those of traceQuery.
+// `Rays` supplies the rays g = first, first + stride, ... < count and takes
+// their results.
+template <bool Full, Query Q, class Rays>
+__device__ __forceinline__ void walkRays(const DevScene& scene, uint32_t count, uint32_t first, uint32_t stride,
+    LdsStack& stack, Rays& rays) {
+    TlasWalk<Full, Q> w;
+    Walk state = Walk::kDone;
+    bool have = false;  // the lane holds a ray
+    uint32_t g = first;
+    rays.begin(g, stride, count);
+    while (true) {
+        bool walking = state == Walk::kTlas, leaf = walking && w.atLeaf();
+        unsigned long long active = __ballot(true), waiting = __ballot(!walking), leaves = __ballot(leaf);
+        int nWait = __popcll(waiting), nLeaf = __popcll(leaves), nAll = __popcll(active);
+        if (nWait < kTraceRefill && nWait != nAll) {
+            int nNode = nAll - nWait - nLeaf;
+            if (nNode >= nLeaf * kLeafWeight) {
+                if (walking && !leaf) state = w.visitNode(scene, stack);
+            } else if (leaf) {
+                state = w.visitLeaf(scene, stack);
+            }
+            continue;
+        }
+        if (walking) continue;
+        if (have) {  // the ray ended
+            if (state == Walk::kAfter) w.finish(scene, stack);
+            rays.done(w.best);
+            g += stride;
+        }
+        if (g >= count) break;
+        Ray ray;
+        float tmax;
+        rays.take(g, stride, count, ray, tmax);
+        state = w.start(scene, ray, tmax, Q == Query::kAny, stack);
+        have = true;
+    }
+}
+
+// The queue's rays, prefetched one ahead.
+struct QueueRays {
+    const LaunchContext& ctx;
+    const SegmentView& v;
+    const PathQueue& q;
+    uint32_t i, nextSlot;
+    Ray next;
+    __device__ void begin(uint32_t g, uint32_t, uint32_t count) {
+        i = nextSlot = 0u;
+        if (g < count) {
+            nextSlot = segmentSlot(v, q.segmentCapacity, g);
+            next = loadRay(q, nextSlot);
+        }
+    }
+    __device__ void take(uint32_t g, uint32_t stride, uint32_t count, Ray& ray, float& tmax) {
+        i = nextSlot;
+        ray = next;
+        tmax = kNoHit;
+        if (g + stride < count) {
+            nextSlot = segmentSlot(v, q.segmentCapacity, g + stride);
+            next = loadRay(q, nextSlot);
+        }
+    }
+    __device__ void done(const HitRecord& h) {
+        ctx.hits.t[i] = h.t;
+        ctx.hits.u[i] = h.u;
+        ctx.hits.v[i] = h.v;
+        ctx.hits.kind[i] = h.kind;
+        ctx.hits.instance[i] = h.instance;
+        ctx.hits.prim[i] = h.prim;
+        ctx.hits.material[i] = h.material;
+    }
+};
 
 // Rays in grid stride: the grid (at most a few times the resident
 // workgroups) bounds the traversal spill area, and the dispatcher balances
@@ -328,45 +410,8 @@ __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kTrace(LaunchContext 
         }
         return;
     }
-    // One loop over node visits, not one per ray: lanes whose rays ended
-    // store their hits and start their next rays (prefetched) while the
-    // other lanes of the wave walk on, once at least kTraceRefill lanes (or
-    // all that are left) wait, instead of idling until every ray of the
-    // wave has ended.
-    TlasWalk<Full, Query::kClosest> w;
-    Walk state = Walk::kDone;
-    bool have = false;  // the lane holds a ray
-    uint32_t g = gid, i = 0;
-    uint32_t nextSlot = g < count ? segmentSlot(v, q.segmentCapacity, g) : 0u;
-    Ray next = g < count ? loadRay(q, nextSlot) : Ray();
-    while (true) {
-        bool walking = state == Walk::kTlas;
-        unsigned long long waiting = __ballot(!walking), left = __ballot(true);
-        if (walking || (__popcll(waiting) < kTraceRefill && waiting != left)) {
-            if (walking) state = w.step(ctx.scene, stack);
-            continue;
-        }
-        if (have) {  // the ray ended: its hit
-            if (state == Walk::kAfter) w.finish(ctx.scene, stack);
-            ctx.hits.t[i] = w.best.t;
-            ctx.hits.u[i] = w.best.u;
-            ctx.hits.v[i] = w.best.v;
-            ctx.hits.kind[i] = w.best.kind;
-            ctx.hits.instance[i] = w.best.instance;
-            ctx.hits.prim[i] = w.best.prim;
-            ctx.hits.material[i] = w.best.material;
-            g += stride;
-        }
-        if (g >= count) break;
-        i = nextSlot;
-        Ray ray = next;
-        if (g + stride < count) {
-            nextSlot = segmentSlot(v, q.segmentCapacity, g + stride);
-            next = loadRay(q, nextSlot);
-        }
-        state = w.start(ctx.scene, ray, kNoHit, false, stack);
-        have = true;
-    }
+    QueueRays rays{ctx, v, q};
+    walkRays<Full, Query::kClosest>(ctx.scene, count, gid, stride, stack, rays);
 }
 
 __device__ __forceinline__ HitRecord loadHit(const HitBuffer& hits, uint32_t i) {
@@ -562,6 +607,48 @@ __global__ void __launch_bounds__(512) WPT_GATHER_OCCUPANCY kGatherEvents(Launch
     }
 }
 
+// The bounce's event rays, prefetched one ahead (the list entry two ahead).
+struct EventRays {
+    const EventBuffer& b;
+    const SegmentView& v;
+    uint32_t i, e, i1, e1, i2, e2;
+    Ray ray1;
+    float tmax1;
+    __device__ void entry(uint32_t at, uint32_t& slot, uint32_t& event) const {
+        uint32_t k = segmentSlot(v, b.raySegment, at);
+        slot = b.raySlot[k];
+        event = b.rayEvent[k];
+    }
+    __device__ void fetch() {
+        ray1 = eventRay(b, e1, i1);
+        tmax1 = __uint_as_float(*eventItemWord(b, e1, kEiTmax, i1));
+    }
+    __device__ void begin(uint32_t g, uint32_t stride, uint32_t count) {
+        i = e = i1 = e1 = i2 = e2 = 0u;
+        tmax1 = 0.0f;
+        if (g < count) {
+            entry(g, i1, e1);
+            fetch();
+        }
+        if (g + stride < count) entry(g + stride, i2, e2);
+    }
+    __device__ void take(uint32_t g, uint32_t stride, uint32_t count, Ray& ray, float& tmax) {
+        i = i1;
+        e = e1;
+        ray = ray1;
+        tmax = tmax1;
+        if (g + stride < count) {
+            i1 = i2;
+            e1 = e2;
+            fetch();
+            if (g + 2u * stride < count) entry(g + 2u * stride, i2, e2);
+        }
+    }
+    __device__ void done(const HitRecord& h) {
+        if (h.kind != kHitNone) *eventItemWord(b, e, kEiFlags, i) |= kEventBlocked;
+    }
+};
+
 // The bounce's event rays, one per thread: a blocked ray marks its event.
 template <bool Full>
 __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kShadowEvents(LaunchContext ctx) {
@@ -572,54 +659,8 @@ __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kShadowEvents(LaunchC
     const uint32_t stride = gridDim.x * blockDim.x;
     const EventBuffer& b = ctx.events;
     LdsStack stack = makeStack(ctx.spill, ctx.spillThreads);
-    auto entry = [&](uint32_t at, uint32_t& slot, uint32_t& event) {
-        uint32_t k = segmentSlot(v, b.raySegment, at);
-        slot = b.raySlot[k];
-        event = b.rayEvent[k];
-    };
-    // The walks of a lane's rays interleave with the other lanes' as in
-    // kTrace.  Prefetched: the next ray (its slot, event, ray and distance)
-    // and the list entry after it.
-    uint32_t i1 = 0, e1 = 0, i2 = 0, e2 = 0;
-    Ray ray1;
-    float tmax1 = 0.0f;
-    if (gid < count) {
-        entry(gid, i1, e1);
-        ray1 = eventRay(b, e1, i1);
-        tmax1 = __uint_as_float(*eventItemWord(b, e1, kEiTmax, i1));
-    }
-    if (gid + stride < count) entry(gid + stride, i2, e2);
-    TlasWalk<Full, Query::kAny> w;
-    Walk state = Walk::kDone;
-    bool have = false;  // the lane holds a ray
-    uint32_t g = gid, i = 0, e = 0;
-    while (true) {
-        bool walking = state == Walk::kTlas;
-        unsigned long long waiting = __ballot(!walking), left = __ballot(true);
-        if (walking || (__popcll(waiting) < kTraceRefill && waiting != left)) {
-            if (walking) state = w.step(ctx.scene, stack);
-            continue;
-        }
-        if (have) {  // the ray ended: a blocked ray marks its event
-            if (state == Walk::kAfter) w.finish(ctx.scene, stack);
-            if (w.best.kind != kHitNone) *eventItemWord(b, e, kEiFlags, i) |= kEventBlocked;
-            g += stride;
-        }
-        if (g >= count) break;
-        i = i1;
-        e = e1;
-        Ray ray = ray1;
-        float tmax = tmax1;
-        if (g + stride < count) {
-            i1 = i2;
-            e1 = e2;
-            ray1 = eventRay(b, e1, i1);
-            tmax1 = __uint_as_float(*eventItemWord(b, e1, kEiTmax, i1));
-            if (g + 2u * stride < count) entry(g + 2u * stride, i2, e2);
-        }
-        state = w.start(ctx.scene, ray, tmax, true, stack);
-        have = true;
-    }
+    EventRays rays{b, v};
+    walkRays<Full, Query::kAny>(ctx.scene, count, gid, stride, stack, rays);
 }
 
 // The events of one shaded path, in order: the contributions whose ray was
