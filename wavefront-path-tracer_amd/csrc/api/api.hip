@@ -81,7 +81,23 @@ struct DeviceArena {
     }
 };
 
-Bvh deviceBvhView(const HostBvh& h, const BvhNode* nodes) {
+// The quad nodes of a host-built tree, made on the device from its binary
+// nodes, which only stay for the copy.
+hipError_t uploadQuads(DeviceArena& a, const std::vector<BvhNode>& nodes, const QuadNode** out) {
+    *out = nullptr;
+    if (nodes.empty()) return hipSuccess;
+    DeviceArena binary;
+    const BvhNode* b = nullptr;
+    void* quads = nullptr;
+    hipError_t e = binary.upload(nodes, &b);
+    if (e == hipSuccess) e = a.alloc(sizeof(QuadNode) * nodes.size(), &quads);
+    if (e == hipSuccess) e = collapseQuads(b, static_cast<uint32_t>(nodes.size()), static_cast<QuadNode*>(quads), nullptr);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    *out = static_cast<const QuadNode*>(quads);
+    return e;
+}
+
+Bvh deviceBvhView(const HostBvh& h, const QuadNode* nodes) {
     Bvh b{};
     b.nodes = nodes;
     b.nodeCount = static_cast<uint32_t>(h.nodes.size());
@@ -286,7 +302,7 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         delete s;
         return fail(WPT_ERROR_INVALID_ARGUMENT, err);
     }
-    if (s->host.maxStackDepth > kMaxStackDepth) {
+    if (s->host.maxStackDepth > kMaxTreeDepth) {
         delete s;
         return fail(WPT_ERROR_UNSUPPORTED, "acceleration structure deeper than the traversal stack");
     }
@@ -316,10 +332,17 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         d.directInstanceCount = static_cast<uint32_t>(h.directInstances.size());
         check(a.upload(h.staticTriangles, &d.staticTriangles), "static triangles");
         d.staticCount = static_cast<uint32_t>(h.staticTriangles.size());
-        const BvhNode* nodes = nullptr;
-        check(a.upload(h.tlas.nodes, &nodes), "tlas nodes");
+        const QuadNode* nodes = nullptr;
+        check(uploadQuads(a, h.tlas.nodes, &nodes), "tlas nodes");
         d.tlas = deviceBvhView(h.tlas, nodes);
         check(a.upload(h.tlasLeavesSlot, &d.tlasLeaves), "tlas leaves");
+        std::vector<float4> leafBounds;
+        for (uint32_t leaf : h.tlas.order) {
+            const Aabb& box = h.tlas.primBounds[leaf];
+            leafBounds.push_back(make_float4(box.mn[0], box.mn[1], box.mn[2], 0.0f));
+            leafBounds.push_back(make_float4(box.mx[0], box.mx[1], box.mx[2], 0.0f));
+        }
+        check(a.upload(leafBounds, &d.tlasBounds), "tlas leaf bounds");
         check(a.upload(h.instances, &d.instances), "instances");
         d.instanceCount = static_cast<uint32_t>(h.instances.size());
         std::vector<Blas> blases(h.meshes.size());
@@ -332,8 +355,9 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
             if (mesh.buildOnDevice && status == WPT_OK) {
                 // Device construction straight into the scene's arena.
                 uint32_t n = b.triangleCount;
-                void *nodes = nullptr, *geometry = nullptr, *order = nullptr;
+                void *nodes = nullptr, *quads = nullptr, *geometry = nullptr, *order = nullptr;
                 check(a.alloc(sizeof(BvhNode) * (n - 1), &nodes), "blas nodes");
+                check(a.alloc(sizeof(QuadNode) * (n - 1), &quads), "blas quad nodes");
                 check(a.alloc(sizeof(float4) * 3 * static_cast<size_t>(n), &geometry), "blas geometry");
                 check(a.alloc(sizeof(uint32_t) * n, &order), "blas order");
                 DeviceBlas& rec = s->deviceBlas[m];
@@ -341,11 +365,14 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
                     check(buildTriangleBvh(b.triangles, n, h.bvhSearchRadius, static_cast<BvhNode*>(nodes),
                               static_cast<float4*>(geometry), static_cast<uint32_t*>(order), nullptr, &rec.build),
                         "device BVH build");
+                if (status == WPT_OK)
+                    check(collapseQuads(static_cast<const BvhNode*>(nodes), n - 1, static_cast<QuadNode*>(quads), nullptr),
+                        "quad nodes");
                 rec.nodes = static_cast<const BvhNode*>(nodes);
                 rec.order = static_cast<const uint32_t*>(order);
                 rec.primCount = n;
                 b.bvh = Bvh{};
-                b.bvh.nodes = rec.nodes;
+                b.bvh.nodes = static_cast<const QuadNode*>(quads);
                 b.bvh.nodeCount = n - 1;
                 b.bvh.primCount = n;
                 b.bvh.root = n > 1 ? 0u : (kLeafBit | 0u);
@@ -358,8 +385,8 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
                 deviceBuildMs += rec.build.milliseconds;
                 continue;
             }
-            const BvhNode* bn = nullptr;
-            check(a.upload(mesh.bvh.nodes, &bn), "blas nodes");
+            const QuadNode* bn = nullptr;
+            check(uploadQuads(a, mesh.bvh.nodes, &bn), "blas nodes");
             b.bvh = deviceBvhView(mesh.bvh, bn);
             check(a.upload(mesh.geometry, &f4), "blas geometry");
             b.geometry = f4;
@@ -367,13 +394,14 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         if (h.bvhBuilder == WPT_BVH_BUILDER_DEVICE_PLOC) {
             h.blasBuildMilliseconds = deviceBuildMs;
             h.maxStackDepth = stackDepth(h);
-            if (status == WPT_OK && h.maxStackDepth > kMaxStackDepth)
+            if (status == WPT_OK && h.maxStackDepth > kMaxTreeDepth)
                 status = fail(WPT_ERROR_UNSUPPORTED, "device-built BVH deeper than the traversal stack");
         }
         check(a.upload(blases, &d.blases), "blases");
         d.blasCount = static_cast<uint32_t>(blases.size());
-        check(a.upload(h.flat.nodes, &nodes), "flat nodes");
+        check(uploadQuads(a, h.flat.nodes, &nodes), "flat nodes");
         d.flat = deviceBvhView(h.flat, nodes);
+        d.flatClipped = h.flat.slotBounds.empty() ? 0u : 1u;
         check(a.upload(h.flatWide, &d.flatWide), "flat wide nodes");
         check(a.upload(h.flatGeometry, &f4), "flat geometry");
         d.flatGeometry = f4;

@@ -34,4 +34,8 @@ struct DeviceBvhBuild {
 hipError_t buildTriangleBvh(const TriShade* triangles, uint32_t n, uint32_t radius, BvhNode* nodes,
     float4* geometry, uint32_t* order, hipStream_t stream, DeviceBvhBuild* result);
 
+// The quad nodes of a binary tree of `count` interior nodes (device memory),
+// node for node.
+hipError_t collapseQuads(const BvhNode* nodes, uint32_t count, QuadNode* out, hipStream_t stream);
+
 }  // namespace wpt

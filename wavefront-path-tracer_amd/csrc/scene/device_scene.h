@@ -2,11 +2,12 @@
 //
 // Layout choices for HBM (reference scene model: include/scene/scene.cuh:117-161,
 // geometry.cuh:6-82):
-//  * BVH2 interior nodes are 64 B and carry both children's bounds, so one
-//    aligned 64 B load tests both children (the reference's 32 B nodes with
-//    own bounds cost three node loads per interior visit).  Children are
-//    either interior node indices or kLeafBit|slot.  Single-primitive leaves,
-//    like NexusBVH's BVH2 (device_traversal.cuh:254-255).
+//  * Trees are built binary (BvhNode, 64 B, both children's bounds, built on
+//    the host or the device; single-primitive leaves, like NexusBVH's BVH2,
+//    device_traversal.cuh:254-255) and walked four wide (QuadNode): one
+//    aligned 128 B line -- the L2 line -- tests four children, where the
+//    reference's 32 B nodes with own bounds cost three node loads per binary
+//    visit.  Children are either interior node indices or kLeafBit|slot.
 //  * Triangle positions used by traversal are separate from shading data:
 //    three float4 (v0|original index, v1|material, v2|flags) = 48 B per
 //    triangle in BVH leaf order, instead of the reference's 228 B AoS record.
@@ -21,6 +22,9 @@
 #if !defined(__HIPCC__)
 struct alignas(16) float4 {
     float x, y, z, w;
+};
+struct alignas(16) uint4 {
+    uint32_t x, y, z, w;
 };
 #endif
 
@@ -37,6 +41,21 @@ struct alignas(16) BvhNode {
 };
 static_assert(sizeof(BvhNode) == 64, "BvhNode must be one 64 B chunk");
 
+// Four-wide node, the form the kernels walk: node i holds binary node i's
+// grandchildren (a child that is a leaf stays, and then the largest
+// grandchild is opened once more), in the binary tree's node and slot
+// numbers, so each is made from the binary tree by itself; the nodes that
+// others opened are never reached.  Planes of the four children side by side,
+// 16 B per plane; an unused child (kInvalid) has an empty box.
+constexpr uint32_t kQuadChildren = 4;
+struct alignas(128) QuadNode {
+    float mn[3][kQuadChildren];
+    float mx[3][kQuadChildren];
+    uint32_t child[kQuadChildren];
+    uint32_t pad[kQuadChildren];
+};
+static_assert(sizeof(QuadNode) == 128, "QuadNode must be one 128 B line");
+
 // Eight-wide node of the flat-triangle accelerator WPT_FLAT_WIDE8: the
 // bounds of up to eight children as coordinate arrays, then the children
 // (interior node index, kLeafBit|slot, or kInvalid for an unused child).
@@ -50,7 +69,7 @@ struct alignas(16) WideNode {
 static_assert(sizeof(WideNode) == 256, "WideNode must be 256 B");
 
 struct Bvh {
-    const BvhNode* nodes;
+    const QuadNode* nodes;
     uint32_t nodeCount;  // interior nodes
     uint32_t root;       // 0 when nodeCount > 0, else kLeafBit|0
     uint32_t primCount;  // 0: no BVH
@@ -247,12 +266,15 @@ struct DevScene {
     const TriShade* staticTriangles;
     Bvh tlas;
     const uint32_t* tlasLeaves;  // slot -> (1<<31 | sphere) or instance
+    const float4* tlasBounds;    // slot -> box of the leaf: minimum, maximum
     const Instance* instances;
     const Blas* blases;
     uint32_t instanceCount;
     uint32_t blasCount;
     Bvh flat;
     const WideNode* flatWide;  // non-null: the flat triangles use eight-wide nodes
+    uint32_t flatClipped;      // leaf boxes of `flat` bound clipped parts of their triangles (spatial splits)
+    uint32_t padFlat;
     const float4* flatGeometry;
     const TriShade* flatTriangles;
     uint32_t flatCount;
