@@ -35,6 +35,7 @@
 #include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../../include/wpt.h"
@@ -232,6 +233,7 @@ __global__ void __launch_bounds__(512) kPrimary(LaunchContext ctx) {
     uint32_t count = passPaths(ctx, tile);
     uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid < kSegments) ctx.counters->count[0][gid] = primarySegmentCount(count, ctx.blockSize, gid);
+    if (gid < 64u) ctx.counters->queueCounts[gid] = 0;
     uint32_t sample = ctx.counters->sampleIndex;
     for (uint32_t g = gid; g < count; g += gridDim.x * blockDim.x)
         storePath(ctx.queue[0], primarySlot(g, ctx.blockSize, ctx.queue[0].segmentCapacity),
@@ -388,6 +390,7 @@ template <bool Full>
 __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kTrace(LaunchContext ctx, uint32_t bounce, uint32_t sel) {
     SegmentView v = loadSegments(ctx.counters->count[sel]);
     uint32_t count = v.start[kSegments];
+    if (count <= ctx.tailPaths) return;  // kTail's
     uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid == 0) {
         atomicAdd(&ctx.counters->closestQueries, static_cast<unsigned long long>(count));
@@ -456,6 +459,7 @@ __global__ void __launch_bounds__(512) kShade(LaunchContext ctx, uint32_t sel) {
     __shared__ AppendShared sh;
     SegmentView v = loadSegments(ctx.counters->count[sel]);
     uint32_t count = v.start[kSegments];
+    if (count <= ctx.tailPaths) return;  // kTail's
     // Queue descriptors by value: a dynamic index into the kernel argument
     // makes the compiler copy the whole argument to scratch.
     const PathQueue q = sel ? ctx.queue[1] : ctx.queue[0];
@@ -520,6 +524,7 @@ __global__ void __launch_bounds__(512) WPT_SHADE_OCCUPANCY kShadeEvents(LaunchCo
     __shared__ AppendShared sh;
     SegmentView v = loadSegments(ctx.counters->count[sel]);
     uint32_t count = v.start[kSegments];
+    if (count <= ctx.tailPaths) return;  // kTail's
     const PathQueue q = sel ? ctx.queue[1] : ctx.queue[0];
     const PathQueue next = sel ? ctx.queue[0] : ctx.queue[1];
     const uint32_t seg = blockIdx.x % kSegments;
@@ -703,6 +708,7 @@ __device__ __forceinline__ void resolveEvents(const LaunchContext& ctx, const Se
 __global__ void __launch_bounds__(512) kResolveEvents(LaunchContext ctx, uint32_t sel) {
     SegmentView v = loadSegments(ctx.counters->count[sel]);
     uint32_t count = v.start[kSegments];
+    if (count <= ctx.tailPaths) return;  // kTail's
     for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < count; g += gridDim.x * blockDim.x)
         resolveEvents(ctx, v, sel, g);
 }
@@ -754,6 +760,172 @@ __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kShadow(LaunchContext
 
 __global__ void kAdvance(LaunchContext ctx) {
     if (ctx.tile->advanceSample) ctx.counters->sampleIndex += ctx.tile->samples;
+}
+
+// One bounce of a path in one lane: its closest hit, shading, and the shadow
+// rays of its radiance events (`column` of the event buffer) or its
+// area-light sample.  Returns whether shading continued the path, which an
+// escaping event may still end (outcome.alive).
+template <bool Full, bool Events>
+__device__ __forceinline__ bool bounceInLane(const LaunchContext& ctx, PathState& path, uint32_t column,
+    LdsStack& stack, uint32_t& shadowQueries, ShadeOutcome& outcome) {
+    if constexpr (Full && Events) {
+        // Shading stores its occlusion-dependent additions as
+        // ordered events in this thread's column; the same
+        // traversal call then resolves them one by one.
+        bool shadowQuery = false;
+        Ray ray = path.ray;
+        float tmax = kNoHit;
+        uint32_t eventCount = 0, eventNext = 0;
+        bool eventEnds = false;
+        while (true) {
+            HitRecord h = traceQuery<Full, Query::kEither>(ctx.scene, ray, tmax, shadowQuery, stack);
+            if (shadowQuery) {
+                ++shadowQueries;
+                if (h.kind == kHitNone) {
+                    path.radiance += eventContribution(ctx.events, eventNext, column);
+                    if (*eventItemWord(ctx.events, eventNext, kEiFlags, column) & kEventTerminates)
+                        eventEnds = true;
+                }
+                ++eventNext;
+            } else {
+                EventOcclusion occ{ctx.events, column, 0u, 0u};
+                shadePath<Full>(ctx.scene, path, h, ctx.shade, occ, outcome);
+                eventCount = occ.count < ctx.events.maxEvents ? occ.count : ctx.events.maxEvents;
+            }
+            while (eventNext < eventCount &&
+                !(*eventItemWord(ctx.events, eventNext, kEiFlags, column) & kEventTraced)) {
+                path.radiance += eventContribution(ctx.events, eventNext, column);
+                ++eventNext;
+            }
+            if (eventNext >= eventCount) break;
+            shadowQuery = true;
+            ray = eventRay(ctx.events, eventNext, column);
+            tmax = __uint_as_float(*eventItemWord(ctx.events, eventNext, kEiTmax, column));
+        }
+        const bool continued = outcome.alive;
+        if (eventEnds) outcome.alive = false;
+        return continued;
+    } else if constexpr (Full) {
+        HitRecord h = traceClosest<Full>(ctx.scene, path.ray, stack);
+        InlineOcclusion<LdsStack> occ{stack, 0u};
+        shadePath<Full>(ctx.scene, path, h, ctx.shade, occ, outcome);
+        shadowQueries += occ.queries;
+    } else {
+        // Without the full feature set the area-light sample is
+        // the bounce's only occlusion test and its last radiance
+        // addition: shading defers it, and the same traversal
+        // call then resolves it (as in the regenerating kernel).
+        DeferOcclusion occ;
+        bool shadowQuery = false;
+        Ray ray = path.ray;
+        float tmax = kNoHit;
+        while (true) {
+            HitRecord h = traceQuery<Full, Query::kEither>(ctx.scene, ray, tmax, shadowQuery, stack);
+            if (shadowQuery) {
+                ++shadowQueries;
+                if (h.kind == kHitNone) path.radiance += outcome.shadow.contribution;
+                break;
+            }
+            shadePath<Full>(ctx.scene, path, h, ctx.shade, occ, outcome);
+            if (!outcome.shadow.valid) break;
+            shadowQuery = true;
+            ray = Ray(outcome.shadow.origin, outcome.shadow.direction);
+            tmax = outcome.shadow.tmax;
+        }
+    }
+    return outcome.alive;
+}
+
+// The rest of a pass once few paths are left: each lane takes a queued path
+// through all its remaining bounces.  A bounce of its own waits for its
+// longest ray walk, a serial chain of several hundred node fetches (250 us on
+// the sphere field), however few rays there are; here a path waits for the
+// walks of its own wave only.  Runs instead of the bounce's staged kernels
+// where the queue holds at most ctx.tailPaths paths, and leaves the next queue
+// empty.  Launched ahead of each bounce's kTrace, it also clears the counters
+// that the bounce's kernels append to.
+// Sphere field 1920x1080, 1 sample: the bounces from 97,000 paths on take
+// 1.6 ms here, 2.6 ms staged; a 97x61 tile of 16 samples (95,000 paths) 0.65
+// ms, 1.5 ms staged.  (Walks interleaved as in walkRays, 182 VGPRs: 2.0 and
+// 1.1 ms; its turns lengthen each step of the chain.)
+constexpr uint32_t kTailBounces = 64;  // bounces counted in WavefrontCounters::queueCounts
+
+struct TailShared {
+    uint32_t bounceCounts[kTailBounces];
+    uint32_t closest, shadow;
+    __device__ void countBounce(uint32_t bounce) {
+        if (bounce < kTailBounces) atomicAdd(&bounceCounts[bounce], 1u);
+    }
+};
+
+// The lane's first path among a queue's `count`: where the grid has lanes to
+// spare, paths take every 2nd .. 64th lane only, so that fewer of them share
+// a wave.  kInvalid: none.
+__device__ __forceinline__ uint32_t tailFirst(uint32_t count, uint32_t gid, uint32_t lanes) {
+    uint32_t spread = 0;
+    while (spread < 6u && (count << (spread + 1u)) <= lanes) ++spread;
+    if (gid & ((1u << spread) - 1u)) return kInvalid;
+    return (gid >> spread) < count ? gid >> spread : kInvalid;
+}
+
+// Clears the next queue's counters; whether this kernel runs the queue, and
+// its view.
+__device__ __forceinline__ bool tailBegin(const LaunchContext& ctx, uint32_t sel, uint32_t gid, SegmentView& v,
+    TailShared& sh) {
+    if (gid < kSegments) {
+        ctx.counters->count[sel ^ 1u][gid] = 0;
+        ctx.counters->shadowCount[gid] = 0;
+        ctx.counters->gatherCount[gid] = 0;
+    }
+    v = loadSegments(ctx.counters->count[sel]);
+    if (v.start[kSegments] == 0 || v.start[kSegments] > ctx.tailPaths) return false;
+    if (threadIdx.x < kTailBounces) sh.bounceCounts[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sh.closest = sh.shadow = 0;
+    __syncthreads();
+    return true;
+}
+
+__device__ __forceinline__ void tailEnd(const LaunchContext& ctx, uint32_t closest, uint32_t shadow, TailShared& sh) {
+    if (closest) atomicAdd(&sh.closest, closest);
+    if (shadow) atomicAdd(&sh.shadow, shadow);
+    __syncthreads();
+    if (threadIdx.x < kTailBounces && ctx.profileQueues && sh.bounceCounts[threadIdx.x])
+        atomicAdd(&ctx.counters->queueCounts[threadIdx.x], sh.bounceCounts[threadIdx.x]);
+    if (threadIdx.x == 0) {
+        if (sh.closest) atomicAdd(&ctx.counters->closestQueries, static_cast<unsigned long long>(sh.closest));
+        if (sh.shadow) atomicAdd(&ctx.counters->shadowQueries, static_cast<unsigned long long>(sh.shadow));
+    }
+}
+
+template <bool Full, bool Events>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3))) kTail(LaunchContext ctx, uint32_t bounce,
+    uint32_t sel) {
+    __shared__ TailShared sh;
+    uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+    SegmentView v;
+    if (!tailBegin(ctx, sel, gid, v, sh)) return;
+    const PathQueue q = sel ? ctx.queue[1] : ctx.queue[0];
+    const uint32_t count = v.start[kSegments], stride = gridDim.x * blockDim.x;
+    LdsStack stack = makeStack(ctx.spill, ctx.spillThreads);
+    uint32_t closest = 0, shadow = 0;
+    for (uint32_t g = tailFirst(count, gid, stride); g < count; g += stride) {
+        PathState path = loadPath(q, segmentSlot(v, q.segmentCapacity, g));
+        sh.countBounce(bounce);
+        ++closest;
+        if (!path.active) continue;  // ended by an event of the previous bounce
+        ShadeOutcome outcome;
+        for (uint32_t b = bounce;;) {
+            outcome.alive = false;
+            bool queued = bounceInLane<Full, Events>(ctx, path, g, stack, shadow, outcome);
+            ++b;
+            if (queued) sh.countBounce(b);
+            if (!outcome.alive) break;
+            ++closest;
+        }
+        finishPath(ctx, path.pixel, outcome.isDebug ? outcome.debugColor : path.radiance);
+    }
+    tailEnd(ctx, closest, shadow, sh);
 }
 
 // Persistent kernel: one grid-wide barrier per bounce.  The resident grid
@@ -817,69 +989,7 @@ __global__ void __launch_bounds__(512) WPT_PERSISTENT_OCCUPANCY(Full, Events) kP
             outcome.alive = false;
             if (valid) {
                 path = loadPath(q, segmentSlot(v, q.segmentCapacity, g));
-                if constexpr (Full && Events) {
-                    // Shading stores its occlusion-dependent additions as
-                    // ordered events in this thread's column; the same
-                    // traversal call then resolves them one by one.
-                    bool shadowQuery = false;
-                    Ray ray = path.ray;
-                    float tmax = kNoHit;
-                    uint32_t eventCount = 0, eventNext = 0;
-                    bool eventEnds = false;
-                    while (true) {
-                        HitRecord h = traceQuery<Full, Query::kEither>(ctx.scene, ray, tmax, shadowQuery, stack);
-                        if (shadowQuery) {
-                            ++shadowQueries;
-                            if (h.kind == kHitNone) {
-                                path.radiance += eventContribution(ctx.events, eventNext, gid);
-                                if (*eventItemWord(ctx.events, eventNext, kEiFlags, gid) & kEventTerminates)
-                                    eventEnds = true;
-                            }
-                            ++eventNext;
-                        } else {
-                            EventOcclusion occ{ctx.events, gid, 0u, 0u};
-                            shadePath<Full>(ctx.scene, path, h, ctx.shade, occ, outcome);
-                            eventCount = occ.count < ctx.events.maxEvents ? occ.count : ctx.events.maxEvents;
-                        }
-                        while (eventNext < eventCount &&
-                            !(*eventItemWord(ctx.events, eventNext, kEiFlags, gid) & kEventTraced)) {
-                            path.radiance += eventContribution(ctx.events, eventNext, gid);
-                            ++eventNext;
-                        }
-                        if (eventNext >= eventCount) break;
-                        shadowQuery = true;
-                        ray = eventRay(ctx.events, eventNext, gid);
-                        tmax = __uint_as_float(*eventItemWord(ctx.events, eventNext, kEiTmax, gid));
-                    }
-                    if (eventEnds) outcome.alive = false;
-                } else if constexpr (Full) {
-                    HitRecord h = traceClosest<Full>(ctx.scene, path.ray, stack);
-                    InlineOcclusion<LdsStack> occ{stack, 0u};
-                    shadePath<Full>(ctx.scene, path, h, ctx.shade, occ, outcome);
-                    shadowQueries += occ.queries;
-                } else {
-                    // Without the full feature set the area-light sample is
-                    // the bounce's only occlusion test and its last radiance
-                    // addition: shading defers it, and the same traversal
-                    // call then resolves it (as in the regenerating kernel).
-                    DeferOcclusion occ;
-                    bool shadowQuery = false;
-                    Ray ray = path.ray;
-                    float tmax = kNoHit;
-                    while (true) {
-                        HitRecord h = traceQuery<Full, Query::kEither>(ctx.scene, ray, tmax, shadowQuery, stack);
-                        if (shadowQuery) {
-                            ++shadowQueries;
-                            if (h.kind == kHitNone) path.radiance += outcome.shadow.contribution;
-                            break;
-                        }
-                        shadePath<Full>(ctx.scene, path, h, ctx.shade, occ, outcome);
-                        if (!outcome.shadow.valid) break;
-                        shadowQuery = true;
-                        ray = Ray(outcome.shadow.origin, outcome.shadow.direction);
-                        tmax = outcome.shadow.tmax;
-                    }
-                }
+                bounceInLane<Full, Events>(ctx, path, gid, stack, shadowQueries, outcome);
             }
             bool alive = valid && outcome.alive;
             uint32_t a, unused;
@@ -955,7 +1065,8 @@ namespace {
 
 // One staged sample; `timer` (optional) brackets every launch with events.
 template <class Timer>
-hipError_t stagedSample(const LaunchContext& ctx, hipStream_t stream, Timer&& timer) {
+hipError_t stagedSample(const LaunchContext& context, hipStream_t stream, Timer&& timer) {
+    LaunchContext ctx = context;
     size_t lds = traversalLdsBytes(ctx.blockSize);
     dim3 grid(ctx.gridBlocks), block(ctx.blockSize);
     // The caustic gather adds radiance after the area light's, so a
@@ -965,10 +1076,22 @@ hipError_t stagedSample(const LaunchContext& ctx, hipStream_t stream, Timer&& ti
     // Such scenes shade without tracing when the renderer holds an event
     // buffer (the usual case), and trace inline otherwise.
     const bool eventShading = inlineShadows && full && ctx.events.words != nullptr;
+    // Inline shading (the renderer holds no event buffer) keeps every bounce.
+    const bool tail = !full || eventShading;
+    ctx.tailPaths = tail ? kTailPaths : 0u;
+    dim3 tailGrid(std::min(ctx.gridBlocks, std::max(1u, kTailLanes / ctx.blockSize)));
+    size_t tailLds = stackLdsBytes(ctx.blockSize);
     hipError_t e = timer(0, [&] { hipLaunchKernelGGL(kPrimary, grid, block, 0, stream, ctx); });
     for (uint32_t bounce = 0; e == hipSuccess && bounce < ctx.shade.maxDepth; ++bounce) {
         uint32_t sel = bounce & 1u;
-        e = timer(1, [&] { hipLaunchKernelGGL(kReset, dim3(1), dim3(64), 0, stream, ctx, sel ^ 1u); });
+        e = timer(1, [&] {
+            if (!full)
+                hipLaunchKernelGGL((kTail<false, false>), tailGrid, block, tailLds, stream, ctx, bounce, sel);
+            else if (eventShading)
+                hipLaunchKernelGGL((kTail<true, true>), tailGrid, block, tailLds, stream, ctx, bounce, sel);
+            else
+                hipLaunchKernelGGL(kReset, dim3(1), dim3(64), 0, stream, ctx, sel ^ 1u);
+        });
         if (e == hipSuccess)
             e = timer(2, [&] {
                 if (full)
