@@ -81,6 +81,15 @@ struct DeviceArena {
     }
 };
 
+// Triangles as queryBrute reads them.
+std::vector<float> triangleEdges(const std::vector<TriShade>& triangles) {
+    std::vector<float> e;
+    e.reserve(9 * triangles.size());
+    for (const TriShade& t : triangles)
+        for (const Vec3& v : {t.v0, t.v1 - t.v0, t.v2 - t.v0}) e.insert(e.end(), {v.x, v.y, v.z});
+    return e;
+}
+
 // The quad nodes of a host-built tree, made on the device from its binary
 // nodes, which only stay for the copy.
 hipError_t uploadQuads(DeviceArena& a, const std::vector<BvhNode>& nodes, const QuadNode** out) {
@@ -331,6 +340,7 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         check(a.upload(h.directInstances, &d.directInstances), "direct instances");
         d.directInstanceCount = static_cast<uint32_t>(h.directInstances.size());
         check(a.upload(h.staticTriangles, &d.staticTriangles), "static triangles");
+        check(a.upload(triangleEdges(h.staticTriangles), &d.staticEdges), "static triangle edges");
         d.staticCount = static_cast<uint32_t>(h.staticTriangles.size());
         const QuadNode* nodes = nullptr;
         check(uploadQuads(a, h.tlas.nodes, &nodes), "tlas nodes");
@@ -346,12 +356,16 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         check(a.upload(h.instances, &d.instances), "instances");
         d.instanceCount = static_cast<uint32_t>(h.instances.size());
         std::vector<Blas> blases(h.meshes.size());
+        std::vector<bool> direct(h.meshes.size(), false);  // meshes some query tests without their tree
+        for (uint32_t i : h.directInstances) direct[h.instances[i].mesh] = true;
         double deviceBuildMs = 0.0;
         for (size_t m = 0; m < h.meshes.size(); ++m) {
             const HostMesh& mesh = h.meshes[m];
             Blas& b = blases[m];
             check(a.upload(mesh.triangles, &b.triangles), "mesh triangles");
             b.triangleCount = static_cast<uint32_t>(mesh.triangles.size());
+            if (direct[m] || (mesh.bvh.primCount() == 0 && !mesh.buildOnDevice))
+                check(a.upload(triangleEdges(mesh.triangles), &b.edges), "mesh triangle edges");
             if (mesh.buildOnDevice && status == WPT_OK) {
                 // Device construction straight into the scene's arena.
                 uint32_t n = b.triangleCount;
@@ -406,6 +420,7 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         check(a.upload(h.flatGeometry, &f4), "flat geometry");
         d.flatGeometry = f4;
         check(a.upload(h.flatTriangles, &d.flatTriangles), "flat triangles");
+        if (h.flat.primCount() == 0) check(a.upload(triangleEdges(h.flatTriangles), &d.flatEdges), "flat triangle edges");
         d.flatCount = static_cast<uint32_t>(h.flatTriangles.size());
         check(a.upload(h.materials, &d.materials), "materials");
         d.materialCount = static_cast<uint32_t>(h.materials.size());

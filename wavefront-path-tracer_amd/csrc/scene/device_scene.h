@@ -136,8 +136,9 @@ struct Blas {
     Bvh bvh;
     const float4* geometry;     // BVH slot order, 3 float4 per triangle
     const TriShade* triangles;  // original order
+    const float* edges;         // v0, v1 - v0, v2 - v0 per triangle; null unless some query tests them all
     uint32_t triangleCount;
-    uint32_t pad[3];
+    uint32_t pad;
 };
 
 struct Material {
@@ -264,6 +265,7 @@ struct DevScene {
     uint32_t directInstanceCount;
     uint32_t staticCount;
     const TriShade* staticTriangles;
+    const float* staticEdges;  // v0, v1 - v0, v2 - v0 per triangle
     Bvh tlas;
     const uint32_t* tlasLeaves;  // slot -> (1<<31 | sphere) or instance
     const float4* tlasBounds;    // slot -> box of the leaf: minimum, maximum
@@ -277,6 +279,7 @@ struct DevScene {
     uint32_t padFlat;
     const float4* flatGeometry;
     const TriShade* flatTriangles;
+    const float* flatEdges;  // as staticEdges, without a tree
     uint32_t flatCount;
     uint32_t materialCount;
     const Material* materials;
