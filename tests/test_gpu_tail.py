@@ -66,3 +66,25 @@ def test_batch_passes_on_both_sides(torch_cuda):
         r.render_samples(2, n)
         image, _ = r.framebuffer()
         assert np.array_equal(out, image[:h, :w])
+
+
+def renderer(width=640, height=480, spp=4, **kw):
+    host = wpt.HostScene("cornell-box")
+    scene = wpt.Scene(host.desc(), device=True, owner=host)
+    cfg = wpt.render_config(width, height, spp=spp, max_depth=4, rr_start=3, **kw)
+    return wpt.Renderer(scene, host.camera(width, height), cfg)
+
+
+@pytest.mark.parametrize("width,height,samples", [(1, 1, 1), (31, 17, 2), (512, 256, 1), (512, 257, 1), (640, 480, 3)])
+def test_small_passes_of_a_large_renderer(torch_cuda, width, height, samples):
+    r = renderer()
+    tile = r.render_task(wpt.Task(0, 0, 1, samples, 640 - width, 480 - height, width, height))
+    r.reset()
+    r.render_samples(1, samples)
+    image, n = r.framebuffer()
+    assert n == 1 + samples
+    assert np.array_equal(tile, image[480 - height:, 640 - width:])
+    tiled = renderer(tile=(200, 130))
+    tiled.render_samples(1, samples)
+    again, n = tiled.framebuffer()
+    assert n == 1 + samples and np.array_equal(again, image)

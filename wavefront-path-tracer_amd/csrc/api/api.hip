@@ -175,10 +175,13 @@ namespace {
 
 __global__ void kSetTile(RenderTile* dst, RenderTile tile) { *dst = tile; }
 __global__ void kSetSample(WavefrontCounters* c, uint32_t sample) { c->sampleIndex = sample; }
-__global__ void kClearStats(WavefrontCounters* c) {
-    c->closestQueries = 0;
-    c->shadowQueries = 0;
-    for (int i = 0; i < 64; ++i) c->queueCounts[i] = 0;
+__global__ void kBeginRender(WavefrontCounters* c, uint32_t sample) {
+    c->queueCounts[threadIdx.x] = 0;
+    if (threadIdx.x == 0) {
+        c->closestQueries = 0;
+        c->shadowQueries = 0;
+        c->sampleIndex = sample;
+    }
 }
 __global__ void kClearRect(float* fb, uint32_t width, uint32_t x0, uint32_t y0, uint32_t w, uint32_t h) {
     size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -225,7 +228,7 @@ std::vector<RenderTile> makeTiles(uint32_t width, uint32_t height, uint32_t tw, 
 int ensureGraph(wpt_renderer* r) {
     if (r->config.mode != WPT_MODE_GRAPH || r->exec) return WPT_OK;
     WPT_HIP(hipStreamBeginCapture(r->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t e = enqueueStagedSample(r->ctx, r->stream);
+    hipError_t e = enqueueStagedSample(r->ctx, r->ctx.capacity, r->stream);
     hipGraph_t graph = nullptr;
     hipError_t e2 = hipStreamEndCapture(r->stream, &graph);
     if (e != hipSuccess) {
@@ -250,7 +253,13 @@ int launchTilePass(wpt_renderer* r, const RenderTile& tile) {
         r->tileValid = true;
     }
     if (r->config.mode == WPT_MODE_GRAPH) {
-        WPT_HIP(hipGraphLaunch(r->exec, r->stream));
+        // Passes that kTail runs whole are three launches; the graph holds
+        // every bounce's.
+        uint64_t paths = static_cast<uint64_t>(tile.width) * tile.height * tile.samples;
+        if (paths <= kTailPaths && r->ctx.capacity > kTailPaths && endsInTail(r->ctx))
+            WPT_HIP(enqueueStagedSample(r->ctx, static_cast<uint32_t>(paths), r->stream));
+        else
+            WPT_HIP(hipGraphLaunch(r->exec, r->stream));
     } else {
         WPT_HIP(enqueuePersistentSample(r->ctx, r->stream));
     }
@@ -1067,8 +1076,7 @@ WPT_API int wpt_renderer_reset(wpt_renderer* r) {
         r->ctx.framebuffer, c.width, 0u, 0u, c.width, c.height);
     hipLaunchKernelGGL(kSetSample, dim3(1), dim3(1), 0, r->stream, r->ctx.counters, 0u);
     WPT_HIP(hipGetLastError());
-    WPT_HIP(hipStreamSynchronize(r->stream));
-    return WPT_OK;
+    return WPT_OK;  // every reader of the frame waits for the stream
 }
 
 WPT_API int wpt_renderer_render_samples(wpt_renderer* r, uint32_t first, uint32_t count) {
@@ -1091,8 +1099,7 @@ WPT_API int wpt_renderer_render_samples(wpt_renderer* r, uint32_t first, uint32_
     }
     int status = ensureGraph(r);
     if (status != WPT_OK) return status;
-    hipLaunchKernelGGL(kClearStats, dim3(1), dim3(1), 0, r->stream, r->ctx.counters);
-    hipLaunchKernelGGL(kSetSample, dim3(1), dim3(1), 0, r->stream, r->ctx.counters, first);
+    hipLaunchKernelGGL(kBeginRender, dim3(1), dim3(64), 0, r->stream, r->ctx.counters, first);
     WPT_HIP(hipGetLastError());
     WPT_HIP(hipEventRecord(r->start, r->stream));
     for (uint32_t s = 0; s < count; s += r->ctx.slots) {
@@ -1170,8 +1177,7 @@ WPT_API int wpt_render_task(wpt_renderer* r, const wpt_task* task, float* hostTi
         size_t n = static_cast<size_t>(task->width) * task->height * 3;
         hipLaunchKernelGGL(kClearRect, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, r->stream,
             r->ctx.framebuffer, c.width, task->x, task->y, task->width, task->height);
-        hipLaunchKernelGGL(kClearStats, dim3(1), dim3(1), 0, r->stream, r->ctx.counters);
-        hipLaunchKernelGGL(kSetSample, dim3(1), dim3(1), 0, r->stream, r->ctx.counters, task->sample_start);
+        hipLaunchKernelGGL(kBeginRender, dim3(1), dim3(64), 0, r->stream, r->ctx.counters, task->sample_start);
         WPT_HIP(hipGetLastError());
         for (uint32_t s = 0; s < task->sample_count; s += r->ctx.slots) {
             tile.samples = std::min(r->ctx.slots, task->sample_count - s);
@@ -1203,8 +1209,7 @@ WPT_API int wpt_renderer_profile_kernels(wpt_renderer* r, uint32_t first, uint32
         launches[4] += 1;
         return WPT_OK;
     }
-    hipLaunchKernelGGL(kClearStats, dim3(1), dim3(1), 0, r->stream, r->ctx.counters);
-    hipLaunchKernelGGL(kSetSample, dim3(1), dim3(1), 0, r->stream, r->ctx.counters, first);
+    hipLaunchKernelGGL(kBeginRender, dim3(1), dim3(64), 0, r->stream, r->ctx.counters, first);
     WPT_HIP(hipGetLastError());
     bool persistent = r->config.mode == WPT_MODE_PERSISTENT;
     for (uint32_t s = 0; s < count; s += r->ctx.slots) {

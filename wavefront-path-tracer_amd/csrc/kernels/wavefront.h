@@ -158,6 +158,14 @@ struct LaunchContext {
 constexpr uint32_t kTailPaths = 131072;
 constexpr uint32_t kTailLanes = 256u * 4u * 3u * 64u;
 
+// Whether the staged scheduler runs a context's small queues through kTail:
+// full-feature scenes that shade inline (the renderer holds no event buffer)
+// or without radiance events keep every bounce.
+inline bool endsInTail(const LaunchContext& c) {
+    return !c.scene.fullFeatures ||
+        ((shadesWithInlineShadows(c.scene) || c.shade.photons != nullptr) && c.events.words != nullptr);
+}
+
 // LDS bytes of the traversal stack for a workgroup of `blockSize` lanes.
 inline size_t stackLdsBytes(uint32_t blockSize) { return sizeof(uint2) * kLdsStackEntries * blockSize; }
 
@@ -180,16 +188,17 @@ inline size_t traversalLdsBytes(uint32_t blockSize) {
     return kLdsPerCu / allowed;
 }
 
-// Staged wavefront: records primary + maxDepth x (reset, trace, shade,
-// shadow) + resolve + advance for one pass of the current tile (its
-// `samples` samples) on `stream` (captured once into a hipGraph by the
+// Staged wavefront: records primary + maxDepth x (tail, trace, shade,
+// shadow) + resolve for one pass of the current tile (its `samples` samples,
+// at most `paths` paths; primary, tail and resolve if they are few) on
+// `stream` (with paths = ctx.capacity captured once into a hipGraph by the
 // caller).
-hipError_t enqueueStagedSample(const LaunchContext& ctx, hipStream_t stream);
-// One staged batch pass (ctx.pieces set): primary, maxDepth x (reset, trace,
-// shade, shadow), then the pieces' resolve into ctx.batchOut.
+hipError_t enqueueStagedSample(const LaunchContext& ctx, uint32_t paths, hipStream_t stream);
+// One staged batch pass (ctx.pieces set): as above, then the pieces' resolve
+// into ctx.batchOut.
 hipError_t enqueueStagedBatchPass(const LaunchContext& ctx, hipStream_t stream);
 // Persistent cooperative kernel for one pass of the current tile, then
-// resolve and advance.
+// resolve.
 hipError_t enqueuePersistentSample(const LaunchContext& ctx, hipStream_t stream);
 // Resident workgroups per CU of each kernel at `blockSize`.
 struct Occupancy {

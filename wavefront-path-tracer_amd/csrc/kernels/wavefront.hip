@@ -8,7 +8,7 @@
 //   appendWarpCompacted (queue_compaction.cuh:8-29) ........... blockAppend in
 //                                                               kShade / kPersistent,
 //                                                               kCompactAbi (C ABI)
-//   advanceSampleIndex (renderer.cu:44-48) .................... kAdvance
+//   advanceSampleIndex (renderer.cu:44-48) .................... kResolve
 //   persistentWavefrontTrace (renderer.cu:55-125) ............. kPersistent
 //
 // Traversal stacks live in LDS (kLdsStackEntries per lane, lane-interleaved
@@ -268,6 +268,7 @@ __global__ void __launch_bounds__(512) kResolve(LaunchContext ctx) {
     RenderTile tile = *ctx.tile;
     uint32_t pixels = tile.width * tile.height;
     uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g == 0 && tile.advanceSample) ctx.counters->sampleIndex += tile.samples;
     if (g >= pixels) return;
     uint32_t x, y;
     tilePixel(tile, g, x, y);
@@ -758,10 +759,6 @@ __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kShadow(LaunchContext
         resolveShadow<Full>(ctx, v, sel, g);
 }
 
-__global__ void kAdvance(LaunchContext ctx) {
-    if (ctx.tile->advanceSample) ctx.counters->sampleIndex += ctx.tile->samples;
-}
-
 // One bounce of a path in one lane: its closest hit, shading, and the shadow
 // rays of its radiance events (`column` of the event buffer) or its
 // area-light sample.  Returns whether shading continued the path, which an
@@ -1063,9 +1060,12 @@ inline uint32_t ceilDiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
 namespace {
 
-// One staged sample; `timer` (optional) brackets every launch with events.
+// One staged sample of at most `paths` paths; `timer` (optional) brackets
+// every launch with events.  Where the whole pass goes to kTail, that is the
+// only launch between the primary rays and the resolve: each of the others
+// took 4 us to find its queue empty.
 template <class Timer>
-hipError_t stagedSample(const LaunchContext& context, hipStream_t stream, Timer&& timer) {
+hipError_t stagedSample(const LaunchContext& context, uint32_t paths, hipStream_t stream, Timer&& timer) {
     LaunchContext ctx = context;
     size_t lds = traversalLdsBytes(ctx.blockSize);
     dim3 grid(ctx.gridBlocks), block(ctx.blockSize);
@@ -1076,12 +1076,11 @@ hipError_t stagedSample(const LaunchContext& context, hipStream_t stream, Timer&
     // Such scenes shade without tracing when the renderer holds an event
     // buffer (the usual case), and trace inline otherwise.
     const bool eventShading = inlineShadows && full && ctx.events.words != nullptr;
-    // Inline shading (the renderer holds no event buffer) keeps every bounce.
-    const bool tail = !full || eventShading;
-    ctx.tailPaths = tail ? kTailPaths : 0u;
+    ctx.tailPaths = endsInTail(ctx) ? kTailPaths : 0u;
     dim3 tailGrid(std::min(ctx.gridBlocks, std::max(1u, kTailLanes / ctx.blockSize)));
     size_t tailLds = stackLdsBytes(ctx.blockSize);
     hipError_t e = timer(0, [&] { hipLaunchKernelGGL(kPrimary, grid, block, 0, stream, ctx); });
+    const bool tailOnly = paths <= ctx.tailPaths;
     for (uint32_t bounce = 0; e == hipSuccess && bounce < ctx.shade.maxDepth; ++bounce) {
         uint32_t sel = bounce & 1u;
         e = timer(1, [&] {
@@ -1092,6 +1091,7 @@ hipError_t stagedSample(const LaunchContext& context, hipStream_t stream, Timer&
             else
                 hipLaunchKernelGGL(kReset, dim3(1), dim3(64), 0, stream, ctx, sel ^ 1u);
         });
+        if (tailOnly) break;
         if (e == hipSuccess)
             e = timer(2, [&] {
                 if (full)
@@ -1130,10 +1130,7 @@ hipError_t stagedSample(const LaunchContext& context, hipStream_t stream, Timer&
         e = timer(6, [&] { hipLaunchKernelGGL(kResolvePieces, dim3(blocks > 0 ? blocks : 1u), block, 0, stream, ctx); });
         return e != hipSuccess ? e : hipGetLastError();
     }
-    e = timer(6, [&] { hipLaunchKernelGGL(kResolve, dim3(ctx.resolveBlocks), block, 0, stream, ctx); });
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kAdvance, dim3(1), dim3(1), 0, stream, ctx);
-    return hipGetLastError();
+    return timer(6, [&] { hipLaunchKernelGGL(kResolve, dim3(ctx.resolveBlocks), block, 0, stream, ctx); });
 }
 
 hipError_t launchPersistent(const LaunchContext& ctx, hipStream_t stream) {
@@ -1149,14 +1146,14 @@ hipError_t launchPersistent(const LaunchContext& ctx, hipStream_t stream) {
 }  // namespace
 
 hipError_t enqueueStagedBatchPass(const LaunchContext& ctx, hipStream_t stream) {
-    return stagedSample(ctx, stream, [](int, auto&& launch) {
+    return stagedSample(ctx, ctx.passPaths, stream, [](int, auto&& launch) {
         launch();
         return hipGetLastError();
     });
 }
 
-hipError_t enqueueStagedSample(const LaunchContext& ctx, hipStream_t stream) {
-    return stagedSample(ctx, stream, [](int, auto&& launch) {
+hipError_t enqueueStagedSample(const LaunchContext& ctx, uint32_t paths, hipStream_t stream) {
+    return stagedSample(ctx, paths, stream, [](int, auto&& launch) {
         launch();
         return hipGetLastError();
     });
@@ -1194,7 +1191,6 @@ hipError_t enqueuePersistentSample(const LaunchContext& ctx, hipStream_t stream)
     hipError_t e = launchPersistent(ctx, stream);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kResolve, dim3(ctx.resolveBlocks), dim3(ctx.blockSize), 0, stream, ctx);
-    hipLaunchKernelGGL(kAdvance, dim3(1), dim3(1), 0, stream, ctx);
     return hipGetLastError();
 }
 
@@ -1225,12 +1221,8 @@ hipError_t profileSample(const LaunchContext& ctx, hipStream_t stream, bool pers
         if (e == hipSuccess) e = launchError;
         if (e == hipSuccess)
             e = timer(6, [&] { hipLaunchKernelGGL(kResolve, dim3(ctx.resolveBlocks), dim3(ctx.blockSize), 0, stream, ctx); });
-        if (e == hipSuccess) {
-            hipLaunchKernelGGL(kAdvance, dim3(1), dim3(1), 0, stream, ctx);
-            e = hipGetLastError();
-        }
     } else {
-        e = stagedSample(ctx, stream, timer);
+        e = stagedSample(ctx, ctx.capacity, stream, timer);
     }
     hipError_t s = hipStreamSynchronize(stream);
     if (e == hipSuccess) e = s;
