@@ -1144,6 +1144,18 @@ WPT_API int wpt_renderer_load_framebuffer(wpt_renderer* r, const float* host, ui
     return WPT_OK;
 }
 
+WPT_API int wpt_host_alloc(uint64_t bytes, void** out) {
+    if (!out || bytes == 0) return fail(WPT_ERROR_INVALID_ARGUMENT, "null output or empty block");
+    *out = nullptr;
+    WPT_HIP(hipHostMalloc(out, bytes));
+    return WPT_OK;
+}
+
+WPT_API int wpt_host_free(void* block) {
+    if (block) WPT_HIP(hipHostFree(block));
+    return WPT_OK;
+}
+
 WPT_API int wpt_render_frame(wpt_renderer* r, float* host, uint32_t* sampleCount) {
     if (!r || !host) return fail(WPT_ERROR_INVALID_ARGUMENT, "null argument");
     int s = wpt_renderer_reset(r);
@@ -1845,10 +1857,15 @@ WPT_API int wpt_batch_render(wpt_batch* b, const wpt_batch_task* tasks, uint32_t
     b->last.samples = samples;
     b->last.milliseconds = ms;
     size_t total = 0;
-    for (uint32_t i = 0; i < n; ++i) total += 3ull * tasks[i].tile_width * tasks[i].tile_height;
-    std::vector<float> host(total);
-    if (total) WPT_HIP(hipMemcpy(host.data(), b->out, sizeof(float) * total, hipMemcpyDeviceToHost));
-    for (uint32_t i = 0; i < n; ++i)
+    bool contiguous = true;  // the outputs lie side by side, as on the device
+    for (uint32_t i = 0; i < n; ++i) {
+        contiguous = contiguous && outs[i] == outs[0] + total;
+        total += 3ull * tasks[i].tile_width * tasks[i].tile_height;
+    }
+    std::vector<float> host(contiguous ? 0 : total);
+    float* copied = contiguous && n ? outs[0] : host.data();
+    if (total) WPT_HIP(hipMemcpy(copied, b->out, sizeof(float) * total, hipMemcpyDeviceToHost));
+    for (uint32_t i = 0; i < n && !contiguous; ++i)
         std::memcpy(outs[i], host.data() + offsets[i], sizeof(float) * 3ull * tasks[i].tile_width * tasks[i].tile_height);
     if (latencyMs && n && !staged) {
         std::vector<BatchTaskState> state(n);
