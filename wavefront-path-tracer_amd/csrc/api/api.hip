@@ -1231,7 +1231,7 @@ WPT_API int wpt_renderer_profile_kernels(wpt_renderer* r, uint32_t first, uint32
             tile.samples = std::min(r->ctx.slots, count - s);
             hipLaunchKernelGGL(kSetTile, dim3(1), dim3(1), 0, r->stream, const_cast<RenderTile*>(r->ctx.tile), tile);
             WPT_HIP(hipGetLastError());
-            WPT_HIP(profileSample(r->ctx, r->stream, persistent, kernelMs, launches));
+            WPT_HIP(profileSample(r->ctx, tile.width * tile.height * tile.samples, r->stream, persistent, kernelMs, launches));
         }
     }
     r->tileValid = false;

@@ -188,11 +188,11 @@ inline size_t traversalLdsBytes(uint32_t blockSize) {
     return kLdsPerCu / allowed;
 }
 
-// Staged wavefront: records primary + maxDepth x (tail, trace, shade,
-// shadow) + resolve for one pass of the current tile (its `samples` samples,
-// at most `paths` paths; primary, tail and resolve if they are few) on
-// `stream` (with paths = ctx.capacity captured once into a hipGraph by the
-// caller).
+// Staged wavefront: records begin + maxDepth x (tail, trace, shade, shadow) +
+// resolve for one pass of the current tile on `stream`, or primary, tail and
+// resolve where kTail takes it whole.  `paths`: a pass of at most kTailPaths
+// gives its own number, any other may give ctx.capacity (captured once into a
+// hipGraph by the caller).
 hipError_t enqueueStagedSample(const LaunchContext& ctx, uint32_t paths, hipStream_t stream);
 // One staged batch pass (ctx.pieces set): as above, then the pieces' resolve
 // into ctx.batchOut.
@@ -209,11 +209,12 @@ struct Occupancy {
 // `events`: the full-feature cooperative kernel resolves radiance events
 // (an event buffer exists), else it traces inline.
 hipError_t kernelOccupancy(uint32_t blockSize, bool full, Occupancy* out, bool events = true);
-// One pass of the current tile with every launch bracketed by events:
+// One pass of the current tile (`paths` paths) with every launch bracketed by
+// events:
 // ms/launches accumulate per kernel (0 primary, 1 reset, 2 trace, 3 shade,
 // 4 persistent, 5 shadow, 6 resolve).  Synchronizes the stream.
 constexpr int kProfileSlots = 7;
-hipError_t profileSample(const LaunchContext& ctx, hipStream_t stream, bool persistent, double ms[kProfileSlots],
+hipError_t profileSample(const LaunchContext& ctx, uint32_t paths, hipStream_t stream, bool persistent, double ms[kProfileSlots],
     uint32_t launches[kProfileSlots]);
 
 // ---- batch consumer ---------------------------------------------------

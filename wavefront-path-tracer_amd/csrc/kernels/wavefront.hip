@@ -1,8 +1,8 @@
 // gfx950 wavefront kernels.
 //
 // Reference kernels and their MI355X counterparts:
-//   generatePrimaryRays (src/renderer/renderer.cu:10-42) ...... kPrimary
-//   intersectScene (device_traversal.cuh:1186-1194) ........... kTrace
+//   generatePrimaryRays (src/renderer/renderer.cu:10-42) ...... FreshPaths
+//   intersectScene (device_traversal.cuh:1186-1194) ........... kTracePrimary, kTrace
 //   shadePaths (device_path_shading.cuh:6-173) ................ kShade
 //   isOccluded calls made inside shadePaths ................... kShadow
 //   appendWarpCompacted (queue_compaction.cuh:8-29) ........... blockAppend in
@@ -228,16 +228,46 @@ __device__ __forceinline__ void finishPath(const LaunchContext& ctx, uint32_t ta
     ctx.slotRadiance[i + 2] = v.z;
 }
 
+// The paths of a pass before their first bounce.
+struct FreshPaths {
+    RenderTile tile;
+    uint32_t sample;
+    __device__ __forceinline__ explicit FreshPaths(const LaunchContext& ctx)
+        : tile(ctx.pieces ? RenderTile{} : *ctx.tile), sample(ctx.counters->sampleIndex) {}
+    __device__ __forceinline__ PathState make(const LaunchContext& ctx, uint32_t g) const {
+        return ctx.pieces ? batchPassPath(ctx, g) : passPath(ctx, tile, sample, g);
+    }
+};
+
+__device__ __forceinline__ uint32_t beginPass(const LaunchContext& ctx, uint32_t t) {
+    uint32_t count = passPaths(ctx, ctx.pieces ? RenderTile{} : *ctx.tile);
+    if (t < kSegments) ctx.counters->count[0][t] = primarySegmentCount(count, ctx.blockSize, t);
+    if (t < 64u) ctx.counters->queueCounts[t] = 0;
+    return count;
+}
+
+// Start of a pass: one workgroup.  The paths are made where they are traced
+// and shaded first (kTracePrimary, kShade) and never stored: making one is a
+// few hundred instructions, storing its 80 B and reading them back twice took
+// longer (sphere field 1920x1080, 64 samples: 53.7 -> 50.8 ms; terrain, 16
+// samples: 139.8 -> 135.6 ms).
+__global__ void kBeginPass(LaunchContext ctx) {
+    beginPass(ctx, threadIdx.x);
+    if (threadIdx.x < kSegments) {
+        ctx.counters->count[1][threadIdx.x] = 0;
+        ctx.counters->shadowCount[threadIdx.x] = 0;
+        ctx.counters->gatherCount[threadIdx.x] = 0;
+    }
+}
+
+// The first queue of a pass that kTail runs whole (made in kTail itself, the
+// path's code costs its lanes spills on every bounce).
 __global__ void __launch_bounds__(512) kPrimary(LaunchContext ctx) {
-    RenderTile tile = ctx.pieces ? RenderTile{} : *ctx.tile;
-    uint32_t count = passPaths(ctx, tile);
     uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid < kSegments) ctx.counters->count[0][gid] = primarySegmentCount(count, ctx.blockSize, gid);
-    if (gid < 64u) ctx.counters->queueCounts[gid] = 0;
-    uint32_t sample = ctx.counters->sampleIndex;
+    uint32_t count = beginPass(ctx, gid);
+    FreshPaths fresh(ctx);
     for (uint32_t g = gid; g < count; g += gridDim.x * blockDim.x)
-        storePath(ctx.queue[0], primarySlot(g, ctx.blockSize, ctx.queue[0].segmentCapacity),
-            ctx.pieces ? batchPassPath(ctx, g) : passPath(ctx, tile, sample, g));
+        storePath(ctx.queue[0], primarySlot(g, ctx.blockSize, ctx.queue[0].segmentCapacity), fresh.make(ctx, g));
 }
 
 // End of a batch pass: each piece's tile pixel adds its samples' radiance,
@@ -350,6 +380,16 @@ __device__ __forceinline__ void walkRays(const DevScene& scene, uint32_t count, 
     }
 }
 
+__device__ __forceinline__ void storeHit(const HitBuffer& hits, uint32_t i, const HitRecord& h) {
+    hits.t[i] = h.t;
+    hits.u[i] = h.u;
+    hits.v[i] = h.v;
+    hits.kind[i] = h.kind;
+    hits.instance[i] = h.instance;
+    hits.prim[i] = h.prim;
+    hits.material[i] = h.material;
+}
+
 // The queue's rays, prefetched one ahead.
 struct QueueRays {
     const LaunchContext& ctx;
@@ -373,15 +413,7 @@ struct QueueRays {
             next = loadRay(q, nextSlot);
         }
     }
-    __device__ void done(const HitRecord& h) {
-        ctx.hits.t[i] = h.t;
-        ctx.hits.u[i] = h.u;
-        ctx.hits.v[i] = h.v;
-        ctx.hits.kind[i] = h.kind;
-        ctx.hits.instance[i] = h.instance;
-        ctx.hits.prim[i] = h.prim;
-        ctx.hits.material[i] = h.material;
-    }
+    __device__ void done(const HitRecord& h) { storeHit(ctx.hits, i, h); }
 };
 
 // Rays in grid stride: the grid (at most a few times the resident
@@ -400,22 +432,27 @@ __global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kTrace(LaunchContext 
     const PathQueue& q = ctx.queue[sel];
     const uint32_t stride = gridDim.x * blockDim.x;
     LdsStack stack = makeStack(ctx.spill, ctx.spillThreads);
-    if (bounce == 0) {  // camera rays: coherent, their walks end nearly together
-        for (uint32_t g = gid; g < count; g += stride) {
-            uint32_t i = segmentSlot(v, q.segmentCapacity, g);
-            HitRecord h = traceClosest<Full>(ctx.scene, loadRay(q, i), stack);
-            ctx.hits.t[i] = h.t;
-            ctx.hits.u[i] = h.u;
-            ctx.hits.v[i] = h.v;
-            ctx.hits.kind[i] = h.kind;
-            ctx.hits.instance[i] = h.instance;
-            ctx.hits.prim[i] = h.prim;
-            ctx.hits.material[i] = h.material;
-        }
-        return;
-    }
     QueueRays rays{ctx, v, q};
     walkRays<Full, Query::kClosest>(ctx.scene, count, gid, stride, stack, rays);
+}
+
+// The first bounce.  Camera rays are coherent and their walks end nearly
+// together: one after the other, without the turns of walkRays.
+template <bool Full>
+__global__ void __launch_bounds__(512) WPT_TRACE_OCCUPANCY kTracePrimary(LaunchContext ctx) {
+    SegmentView v = loadSegments(ctx.counters->count[0]);
+    uint32_t count = v.start[kSegments];
+    uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid == 0) {
+        atomicAdd(&ctx.counters->closestQueries, static_cast<unsigned long long>(count));
+        if (ctx.profileQueues) ctx.counters->queueCounts[0] = count;
+    }
+    LdsStack stack = makeStack(ctx.spill, ctx.spillThreads);
+    FreshPaths fresh(ctx);
+    for (uint32_t g = gid; g < count; g += gridDim.x * blockDim.x) {
+        HitRecord h = traceClosest<Full>(ctx.scene, fresh.make(ctx, g).ray, stack);
+        storeHit(ctx.hits, primarySlot(g, ctx.blockSize, ctx.queue[0].segmentCapacity), h);
+    }
 }
 
 __device__ __forceinline__ HitRecord loadHit(const HitBuffer& hits, uint32_t i) {
@@ -456,16 +493,18 @@ __device__ __forceinline__ void storeShadow(const ShadowQueue& q, uint32_t s, co
 // or punctual lights, whose shading adds radiance after the area-light NEE)
 // every shadow ray is traced here and the shadow queue stays empty.
 template <bool Inline, bool Full>
-__global__ void __launch_bounds__(512) kShade(LaunchContext ctx, uint32_t sel) {
+__global__ void __launch_bounds__(512) kShade(LaunchContext ctx, uint32_t bounce) {
     __shared__ AppendShared sh;
+    const uint32_t sel = bounce & 1u;
     SegmentView v = loadSegments(ctx.counters->count[sel]);
     uint32_t count = v.start[kSegments];
-    if (count <= ctx.tailPaths) return;  // kTail's
+    if (bounce && count <= ctx.tailPaths) return;  // kTail's
     // Queue descriptors by value: a dynamic index into the kernel argument
     // makes the compiler copy the whole argument to scratch.
     const PathQueue q = sel ? ctx.queue[1] : ctx.queue[0];
     const PathQueue next = sel ? ctx.queue[0] : ctx.queue[1];
     const uint32_t seg = blockIdx.x % kSegments;
+    const FreshPaths fresh(ctx);
     for (uint32_t first = blockIdx.x * blockDim.x; first < count; first += gridDim.x * blockDim.x) {
         uint32_t g = first + threadIdx.x;
         bool valid = g < count;
@@ -474,8 +513,8 @@ __global__ void __launch_bounds__(512) kShade(LaunchContext ctx, uint32_t sel) {
         outcome.alive = false;
         outcome.shadow.valid = 0;
         if (valid) {
-            uint32_t i = segmentSlot(v, q.segmentCapacity, g);
-            path = loadPath(q, i);
+            uint32_t i = bounce ? segmentSlot(v, q.segmentCapacity, g) : primarySlot(g, ctx.blockSize, q.segmentCapacity);
+            path = bounce ? loadPath(q, i) : fresh.make(ctx, g);
             if constexpr (Inline) {
                 LdsStack stack = makeStack(ctx.spill, ctx.spillThreads);
                 InlineOcclusion<LdsStack> occ{stack, 0u};
@@ -521,15 +560,17 @@ __device__ __forceinline__ Ray eventRay(const EventBuffer& b, uint32_t e, uint32
 // kResolveEvents completes the radiance.  Paths without events finish or
 // continue here as in kShade.
 template <bool Full>
-__global__ void __launch_bounds__(512) WPT_SHADE_OCCUPANCY kShadeEvents(LaunchContext ctx, uint32_t sel) {
+__global__ void __launch_bounds__(512) WPT_SHADE_OCCUPANCY kShadeEvents(LaunchContext ctx, uint32_t bounce) {
     __shared__ AppendShared sh;
+    const uint32_t sel = bounce & 1u;
     SegmentView v = loadSegments(ctx.counters->count[sel]);
     uint32_t count = v.start[kSegments];
-    if (count <= ctx.tailPaths) return;  // kTail's
+    if (bounce && count <= ctx.tailPaths) return;  // kTail's
     const PathQueue q = sel ? ctx.queue[1] : ctx.queue[0];
     const PathQueue next = sel ? ctx.queue[0] : ctx.queue[1];
     const uint32_t seg = blockIdx.x % kSegments;
     const uint32_t maxEvents = ctx.events.maxEvents;
+    const FreshPaths fresh(ctx);
     for (uint32_t first = blockIdx.x * blockDim.x; first < count; first += gridDim.x * blockDim.x) {
         uint32_t g = first + threadIdx.x;
         bool valid = g < count;
@@ -539,8 +580,8 @@ __global__ void __launch_bounds__(512) WPT_SHADE_OCCUPANCY kShadeEvents(LaunchCo
         outcome.alive = false;
         outcome.isDebug = false;
         if (valid) {
-            i = segmentSlot(v, q.segmentCapacity, g);
-            path = loadPath(q, i);
+            i = bounce ? segmentSlot(v, q.segmentCapacity, g) : primarySlot(g, ctx.blockSize, q.segmentCapacity);
+            path = bounce ? loadPath(q, i) : fresh.make(ctx, g);
             if (path.active) {
                 StagedEventOcclusion occ{{ctx.events, i, 0u, 0u}, 0u};
                 shadePath<Full>(ctx.scene, path, loadHit(ctx.hits, i), ctx.shade, occ, outcome);
@@ -1079,22 +1120,32 @@ hipError_t stagedSample(const LaunchContext& context, uint32_t paths, hipStream_
     ctx.tailPaths = endsInTail(ctx) ? kTailPaths : 0u;
     dim3 tailGrid(std::min(ctx.gridBlocks, std::max(1u, kTailLanes / ctx.blockSize)));
     size_t tailLds = stackLdsBytes(ctx.blockSize);
-    hipError_t e = timer(0, [&] { hipLaunchKernelGGL(kPrimary, grid, block, 0, stream, ctx); });
     const bool tailOnly = paths <= ctx.tailPaths;
+    hipError_t e = timer(0, [&] {
+        if (tailOnly)
+            hipLaunchKernelGGL(kPrimary, grid, block, 0, stream, ctx);
+        else
+            hipLaunchKernelGGL(kBeginPass, dim3(1), dim3(64), 0, stream, ctx);
+    });
     for (uint32_t bounce = 0; e == hipSuccess && bounce < ctx.shade.maxDepth; ++bounce) {
         uint32_t sel = bounce & 1u;
-        e = timer(1, [&] {
-            if (!full)
-                hipLaunchKernelGGL((kTail<false, false>), tailGrid, block, tailLds, stream, ctx, bounce, sel);
-            else if (eventShading)
-                hipLaunchKernelGGL((kTail<true, true>), tailGrid, block, tailLds, stream, ctx, bounce, sel);
-            else
-                hipLaunchKernelGGL(kReset, dim3(1), dim3(64), 0, stream, ctx, sel ^ 1u);
-        });
+        if (bounce || tailOnly)
+            e = timer(1, [&] {
+                if (!full)
+                    hipLaunchKernelGGL((kTail<false, false>), tailGrid, block, tailLds, stream, ctx, bounce, sel);
+                else if (eventShading)
+                    hipLaunchKernelGGL((kTail<true, true>), tailGrid, block, tailLds, stream, ctx, bounce, sel);
+                else
+                    hipLaunchKernelGGL(kReset, dim3(1), dim3(64), 0, stream, ctx, sel ^ 1u);
+            });
         if (tailOnly) break;
         if (e == hipSuccess)
             e = timer(2, [&] {
-                if (full)
+                if (bounce == 0 && full)
+                    hipLaunchKernelGGL(kTracePrimary<true>, grid, block, lds, stream, ctx);
+                else if (bounce == 0)
+                    hipLaunchKernelGGL(kTracePrimary<false>, grid, block, lds, stream, ctx);
+                else if (full)
                     hipLaunchKernelGGL(kTrace<true>, grid, block, lds, stream, ctx, bounce, sel);
                 else
                     hipLaunchKernelGGL(kTrace<false>, grid, block, lds, stream, ctx, bounce, sel);
@@ -1102,13 +1153,13 @@ hipError_t stagedSample(const LaunchContext& context, uint32_t paths, hipStream_
         if (e == hipSuccess)
             e = timer(3, [&] {
                 if (eventShading)
-                    hipLaunchKernelGGL(kShadeEvents<true>, grid, block, 0, stream, ctx, sel);
+                    hipLaunchKernelGGL(kShadeEvents<true>, grid, block, 0, stream, ctx, bounce);
                 else if (inlineShadows)
-                    hipLaunchKernelGGL((kShade<true, true>), grid, block, lds, stream, ctx, sel);
+                    hipLaunchKernelGGL((kShade<true, true>), grid, block, lds, stream, ctx, bounce);
                 else if (full)
-                    hipLaunchKernelGGL((kShade<false, true>), grid, block, 0, stream, ctx, sel);
+                    hipLaunchKernelGGL((kShade<false, true>), grid, block, 0, stream, ctx, bounce);
                 else
-                    hipLaunchKernelGGL((kShade<false, false>), grid, block, 0, stream, ctx, sel);
+                    hipLaunchKernelGGL((kShade<false, false>), grid, block, 0, stream, ctx, bounce);
             });
         if (e == hipSuccess && eventShading && ctx.shade.photons)
             e = timer(3, [&] { hipLaunchKernelGGL(kGatherEvents, grid, block, 0, stream, ctx); });
@@ -1194,7 +1245,7 @@ hipError_t enqueuePersistentSample(const LaunchContext& ctx, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t profileSample(const LaunchContext& ctx, hipStream_t stream, bool persistent, double ms[kProfileSlots],
+hipError_t profileSample(const LaunchContext& ctx, uint32_t paths, hipStream_t stream, bool persistent, double ms[kProfileSlots],
     uint32_t launches[kProfileSlots]) {
     struct Span {
         int kind;
@@ -1222,7 +1273,7 @@ hipError_t profileSample(const LaunchContext& ctx, hipStream_t stream, bool pers
         if (e == hipSuccess)
             e = timer(6, [&] { hipLaunchKernelGGL(kResolve, dim3(ctx.resolveBlocks), dim3(ctx.blockSize), 0, stream, ctx); });
     } else {
-        e = stagedSample(ctx, ctx.capacity, stream, timer);
+        e = stagedSample(ctx, paths, stream, timer);
     }
     hipError_t s = hipStreamSynchronize(stream);
     if (e == hipSuccess) e = s;
