@@ -92,3 +92,55 @@ def test_non_finite_rays_hit_nothing(torch_cuda):
     hits = trav.gpu_trace(torch_cuda, scene, rays)
     assert np.all(hits["kind"] == wpt.HIT_NONE)
     assert not trav.gpu_occluded(torch_cuda, scene, rays, np.full(rays.shape[1], 10.0, np.float32)).any()
+
+
+def bumpy_grid(n, bump, seed):
+    """An n x n grid of unit cells whose heights vary by `bump`, as vertices."""
+    h = np.random.default_rng(seed).uniform(-bump, bump, (n + 1, n + 1)) if bump else np.zeros((n + 1, n + 1))
+    tris = []
+    for i in range(n):
+        for k in range(n):
+            a, b, c, d = ((x - n / 2, h[x, z], z - n / 2) for x, z in ((i, k), (i + 1, k), (i + 1, k + 1), (i, k + 1)))
+            tris += [(a, b, c), (a, c, d)]
+    return np.array(tris, np.float32)
+
+
+def aimed_rays(verts, n, seed):
+    """Rays at points of the triangles' edges, more than half of them grazing."""
+    rng = np.random.default_rng(seed)
+    tri = verts[rng.integers(0, len(verts), n)].astype(np.float64)
+    e, s = rng.integers(0, 3, n), rng.random((n, 1))
+    a, b = tri[np.arange(n), e], tri[np.arange(n), (e + 1) % 3]
+    d = rng.normal(size=(n, 3))
+    graze = rng.random(n) < 0.6
+    d[graze, 1] *= np.exp(rng.uniform(np.log(1e-5), 0, graze.sum()))
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    origin = (a + (b - a) * s - d * np.exp(rng.uniform(np.log(0.05), np.log(600.0), (n, 1)))).astype(np.float32)
+    d = a + (b - a) * s - origin
+    d /= np.maximum(np.linalg.norm(d, axis=1), 1e-30)[:, None]
+    return np.concatenate([origin.T, d.T]).astype(np.float32)
+
+
+@pytest.mark.parametrize("accel", [wpt.FLAT_SAH_BVH2, wpt.FLAT_MEDIAN_BVH2, wpt.FLAT_SPATIAL_SPLIT_BVH2])
+@pytest.mark.parametrize("bump", [0.0, 0.3])
+def test_rays_at_edges_of_flat_trees(torch_cuda, oracle_mod, accel, bump):
+    """What is hit, and on the flat grid (where every distance is the plane's)
+    which triangle.  On the bumpy grid a triangle hit a few ulps outside its
+    box counts or not by the order in which the tree is walked, where boxes
+    overlap (median and split trees): its neighbour is then hit instead, at
+    nearly the same distance."""
+    verts = bumpy_grid(40, bump, 3)
+    b = wpt.SceneBuilder()
+    b.material(wpt.make_material(wpt.DIFFUSE, (0.5, 0.5, 0.5)))
+    b.flat_triangles = [wpt.make_triangle(*t.tolist(), 0) for t in verts]
+    b.flat_accelerator = accel
+    scene = wpt.Scene(b.desc(), device=True, owner=b)
+    oracle, rays = oracle_mod.Oracle(scene), aimed_rays(verts, 400000, 1)
+    if bump == 0.0 or accel == wpt.FLAT_SAH_BVH2:
+        check(torch_cuda, oracle, scene, f"accelerator {accel}, bump {bump}", rays)
+        return
+    want, got = oracle.trace(rays), trav.gpu_trace(torch_cuda, scene, rays)
+    assert np.array_equal(got["kind"], want["kind"])
+    assert np.allclose(got["t"], want["t"], rtol=1e-3)
+    for p, q in zip(*(h["primitive"][got["primitive"] != want["primitive"]] for h in (got, want))):
+        assert len(set(map(tuple, verts[p])) & set(map(tuple, verts[q]))) > 0, (p, q)

@@ -90,6 +90,14 @@ std::vector<float> triangleEdges(const std::vector<TriShade>& triangles) {
     return e;
 }
 
+// Leaf boxes as slotOpen reads them.
+void appendBoxes(std::vector<float4>& out, const std::vector<Aabb>& boxes) {
+    for (const Aabb& b : boxes) {
+        out.push_back(make_float4(b.mn[0], b.mn[1], b.mn[2], 0.0f));
+        out.push_back(make_float4(b.mx[0], b.mx[1], b.mx[2], 0.0f));
+    }
+}
+
 // The quad nodes of a host-built tree, made on the device from its binary
 // nodes, which only stay for the copy.
 hipError_t uploadQuads(DeviceArena& a, const std::vector<BvhNode>& nodes, const QuadNode** out) {
@@ -355,12 +363,10 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         check(uploadQuads(a, h.tlas.nodes, &nodes), "tlas nodes");
         d.tlas = deviceBvhView(h.tlas, nodes);
         check(a.upload(h.tlasLeavesSlot, &d.tlasLeaves), "tlas leaves");
+        std::vector<Aabb> leafBoxes;
+        for (uint32_t leaf : h.tlas.order) leafBoxes.push_back(h.tlas.primBounds[leaf]);
         std::vector<float4> leafBounds;
-        for (uint32_t leaf : h.tlas.order) {
-            const Aabb& box = h.tlas.primBounds[leaf];
-            leafBounds.push_back(make_float4(box.mn[0], box.mn[1], box.mn[2], 0.0f));
-            leafBounds.push_back(make_float4(box.mx[0], box.mx[1], box.mx[2], 0.0f));
-        }
+        appendBoxes(leafBounds, leafBoxes);
         check(a.upload(leafBounds, &d.tlasBounds), "tlas leaf bounds");
         check(a.upload(h.instances, &d.instances), "instances");
         d.instanceCount = static_cast<uint32_t>(h.instances.size());
@@ -426,7 +432,9 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
         d.flat = deviceBvhView(h.flat, nodes);
         d.flatClipped = h.flat.slotBounds.empty() ? 0u : 1u;
         check(a.upload(h.flatWide, &d.flatWide), "flat wide nodes");
-        check(a.upload(h.flatGeometry, &f4), "flat geometry");
+        std::vector<float4> flatGeometry = h.flatGeometry;
+        appendBoxes(flatGeometry, h.flat.slotBounds);
+        check(a.upload(flatGeometry, &f4), "flat geometry");
         d.flatGeometry = f4;
         check(a.upload(h.flatTriangles, &d.flatTriangles), "flat triangles");
         if (h.flat.primCount() == 0) check(a.upload(triangleEdges(h.flatTriangles), &d.flatEdges), "flat triangle edges");

@@ -277,7 +277,7 @@ struct DevScene {
     const WideNode* flatWide;  // non-null: the flat triangles use eight-wide nodes
     uint32_t flatClipped;      // leaf boxes of `flat` bound clipped parts of their triangles (spatial splits)
     uint32_t padFlat;
-    const float4* flatGeometry;
+    const float4* flatGeometry;  // slot order, 3 float4 per triangle; if clipped, then 2 per leaf box
     const TriShade* flatTriangles;
     const float* flatEdges;  // as staticEdges, without a tree
     uint32_t flatCount;
