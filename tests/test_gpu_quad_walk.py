@@ -121,7 +121,8 @@ def aimed_rays(verts, n, seed):
     return np.concatenate([origin.T, d.T]).astype(np.float32)
 
 
-@pytest.mark.parametrize("accel", [wpt.FLAT_SAH_BVH2, wpt.FLAT_MEDIAN_BVH2, wpt.FLAT_SPATIAL_SPLIT_BVH2])
+@pytest.mark.parametrize("accel", [wpt.FLAT_SAH_BVH2, wpt.FLAT_MEDIAN_BVH2, wpt.FLAT_SPATIAL_SPLIT_BVH2,
+                                   wpt.FLAT_WIDE8])
 @pytest.mark.parametrize("bump", [0.0, 0.3])
 def test_rays_at_edges_of_flat_trees(torch_cuda, oracle_mod, accel, bump):
     """What is hit, and on the flat grid (where every distance is the plane's)
@@ -136,7 +137,7 @@ def test_rays_at_edges_of_flat_trees(torch_cuda, oracle_mod, accel, bump):
     b.flat_accelerator = accel
     scene = wpt.Scene(b.desc(), device=True, owner=b)
     oracle, rays = oracle_mod.Oracle(scene), aimed_rays(verts, 400000, 1)
-    if bump == 0.0 or accel == wpt.FLAT_SAH_BVH2:
+    if bump == 0.0 or accel in (wpt.FLAT_SAH_BVH2, wpt.FLAT_WIDE8):
         check(torch_cuda, oracle, scene, f"accelerator {accel}, bump {bump}", rays)
         return
     want, got = oracle.trace(rays), trav.gpu_trace(torch_cuda, scene, rays)

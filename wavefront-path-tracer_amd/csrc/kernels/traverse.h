@@ -272,14 +272,15 @@ struct PrivateStack {
     }
 };
 
-// Pops until an entry still closer than closestT; false when the traversal
-// level (entries above `base`) is exhausted.
+// Pops until an entry within `reach`, the reach of the box test that pushed
+// the entries: boxReach(closestT), or tieReach(closestT) for slab() alone;
+// false when the traversal level (entries above `base`) is exhausted.
 template <class Stack>
-WPT_HD bool popLive(Stack& stack, uint32_t base, float closestT, uint32_t& cur) {
+WPT_HD bool popLive(Stack& stack, uint32_t base, float reach, uint32_t& cur) {
     while (stack.size > base) {
         float t;
         stack.pop(cur, t);
-        if (t <= boxReach(closestT)) return true;
+        if (t <= reach) return true;
     }
     return false;
 }
@@ -421,7 +422,7 @@ WPT_HD bool queryBvh(const DevScene& s, const RayInv& r, const Bvh& bvh, const f
         } else {
             if (visitQuad(bvh.nodes, b, best.t, cur, stack)) continue;
         }
-        if (!popLive(stack, base, best.t, cur)) return false;
+        if (!popLive(stack, base, boxReach(best.t), cur)) return false;
     }
 }
 
@@ -476,7 +477,7 @@ WPT_HD bool queryWide(const DevScene& s, const RayInv& r, const Bvh& bvh, const 
                 ++pushed;
             }
         }
-        if (!popLive(stack, base, best.t, cur)) return false;
+        if (!popLive(stack, base, tieReach(best.t), cur)) return false;
     }
 }
 
@@ -620,12 +621,12 @@ struct TlasWalk {
     template <class Stack>
     WPT_HD Walk next(const DevScene& s, Stack& stack) {
         if (instance != kInvalid) {
-            if (popLive(stack, blasBase, best.t, cur)) return Walk::kTlas;
+            if (popLive(stack, blasBase, boxReach(best.t), cur)) return Walk::kTlas;
             instance = kInvalid;
             nodes = s.tlas.nodes;
             r = makeBoxRay(ray, worldInv);
         }
-        return popLive(stack, base, best.t, cur) ? Walk::kTlas : Walk::kAfter;
+        return popLive(stack, base, boxReach(best.t), cur) ? Walk::kTlas : Walk::kAfter;
     }
 
     WPT_HD bool atLeaf() const { return (cur & kLeafBit) != 0u; }
@@ -802,12 +803,12 @@ WPT_HD HitRecord traceQuery(const DevScene& s, const Ray& ray, float maxDistance
                     if (visitQuad(nodes, r, best.t, cur, stack)) continue;
                 }
                 if (instance != kInvalid) {
-                    if (popLive(stack, blasBase, best.t, cur)) continue;
+                    if (popLive(stack, blasBase, boxReach(best.t), cur)) continue;
                     instance = kInvalid;
                     nodes = s.tlas.nodes;
                     r = makeBoxRay(ray, worldInv);
                 }
-                if (!popLive(stack, base, best.t, cur)) break;
+                if (!popLive(stack, base, boxReach(best.t), cur)) break;
             }
         }
     }
