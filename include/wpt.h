@@ -478,7 +478,8 @@ WPT_API int wpt_renderer_read_framebuffer(wpt_renderer* renderer, float* host_rg
  * loadRenderSessionCheckpoint, render_checkpoint.cpp:187-192). */
 WPT_API int wpt_renderer_load_framebuffer(wpt_renderer* renderer, const float* host_rgb, uint32_t sample_count);
 /* Page-locked host memory: results are read back into it at the link's rate,
- * without staging copies and page faults.  Free with wpt_host_free. */
+ * without staging copies and page faults.  Not mapped in a forked process.
+ * Free with wpt_host_free, not while a stream of the caller's is captured. */
 WPT_API int wpt_host_alloc(uint64_t bytes, void** out);
 WPT_API int wpt_host_free(void* block);
 /* Full render: reset + all spp + read back (RenderDriver::run). */

@@ -1,6 +1,9 @@
-"""Results read back into page-locked blocks: arrays stay what they were while
-their owner renders on, however many are held, also after it is closed."""
+"""Results are ordinary arrays with memory of their own: they stay what they
+were while their owner renders on, however many are held, also after it is
+closed, and a forked process has them too."""
+import ctypes as C
 import gc
+import threading
 
 import numpy as np
 import pytest
@@ -56,3 +59,59 @@ def test_batch_results_are_separate(torch_cuda):
     assert np.array_equal(first[0], keep[0]) and np.array_equal(first[2], keep[2])
     assert all(np.array_equal(a, b) for a, b in zip(second, keep[::-1]))
     assert batch.render([]) == []
+
+
+def map_flags(array):
+    """The flags of the memory mappings that hold the array's first and last byte."""
+    flags, ends = [], (array.ctypes.data, array.ctypes.data + array.nbytes - 1)
+    for line in open("/proc/self/smaps"):
+        word = line.split(" ")[0]
+        if "-" in word and ":" not in word:
+            lo, hi = (int(x, 16) for x in word.split("-"))
+            held = any(lo <= end < hi for end in ends)
+        elif word == "VmFlags:" and held:
+            flags += line.split()[1:]
+    assert flags
+    return flags
+
+
+@pytest.mark.parametrize("width,height", [(64, 48), (640, 480), (1500, 700)])
+def test_result_memory_is_the_callers(torch_cuda, width, height):
+    r = renderer(width, height, spp=1)
+    frame, _ = r.render_frame()
+    r.render_samples(1, 1)
+    again, _ = r.framebuffer()
+    tile = r.render_task(wpt.Task(0, 0, 0, 1, 3, 5, width - 3, height - 5))
+    host = wpt.HostScene("cornell-box")
+    scene = wpt.Scene(host.desc(), device=True, owner=host)
+    tasks = [wpt.batch_task(0, host.camera(width, height), width, height, x, 0, w, height, 0, 1, max_depth=4)
+             for x, w in ((0, 1), (1, width // 2), (40, 24))]
+    for a in [frame, again, tile] + wpt.Batch([scene]).render(tasks):
+        assert a.base is None  # keeping one result keeps no other
+        flags = map_flags(a)
+        assert "dc" not in flags and "sh" not in flags, flags  # copied on fork
+
+
+@pytest.mark.parametrize("width,height", [(418, 418), (419, 418), (836, 418), (1277, 719)])
+def test_whole_frames_from_several_threads(torch_cuda, width, height):
+    """Frames just below and above the size read in pieces, of one piece and
+    of several with a remainder, into ordinary and page-locked memory."""
+    r = renderer(width, height, spp=1)
+    r.render_samples(0, 1)
+    want = r.render_task(wpt.Task(0, 0, 0, 1, 0, 0, width, height))
+    got = [None] * 4
+
+    def read(k):
+        got[k] = r.framebuffer()[0]
+
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(len(got))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    lib, block = wpt.library(), C.c_void_p()
+    wpt.check(lib.wpt_host_alloc(want.nbytes, C.byref(block)), "wpt_host_alloc")
+    wpt.check(lib.wpt_renderer_read_framebuffer(r._h, block, None), "wpt_renderer_read_framebuffer")
+    locked = np.ctypeslib.as_array(C.cast(block, C.POINTER(C.c_float)), want.shape).copy()
+    wpt.check(lib.wpt_host_free(block), "wpt_host_free")
+    assert all(np.array_equal(g, want) for g in got + [locked])

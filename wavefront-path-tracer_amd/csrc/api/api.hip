@@ -81,6 +81,90 @@ struct DeviceArena {
     }
 };
 
+// Device results on their way into ordinary host memory: through two
+// page-locked halves of fixed size, the link filling one while the CPU empties
+// the other.  A 1080p framebuffer (25 MB) into memory that is already mapped
+// takes 990 us so, 1380 us by one hipMemcpy, whose staging takes turns with its
+// transfers (into page-locked memory, 470 us; halves of 1 to 4 MiB alike).  One
+// hipMemcpy2D of a 97x61 tile into ordinary memory makes its task 664 us, where
+// rows that land in page-locked memory make it 313.
+class ReadBack {
+    static constexpr size_t kHalf = size_t(1) << 21;
+    std::mutex mutex;  // reads of one owner may come from several threads
+    char* block = nullptr;
+    hipEvent_t filled[2] = {nullptr, nullptr};
+
+    // Piece k by fill(k, half), then take(k, half) once it is there.
+    template <class Fill, class Take>
+    hipError_t pump(size_t pieces, hipStream_t stream, Fill&& fill, Take&& take) {
+        std::lock_guard<std::mutex> lock(mutex);
+        auto start = [&](size_t k) {
+            hipError_t e = fill(k, block + (k & 1) * kHalf);
+            return e == hipSuccess ? hipEventRecord(filled[k & 1], stream) : e;
+        };
+        hipError_t e = pieces ? start(0) : hipSuccess;
+        for (size_t k = 0; e == hipSuccess && k < pieces; ++k) {
+            if (k + 1 < pieces) e = start(k + 1);
+            if (e == hipSuccess) e = hipEventSynchronize(filled[k & 1]);
+            if (e == hipSuccess) take(k, block + (k & 1) * kHalf);
+        }
+        return e;
+    }
+
+public:
+    static bool worthwhile(size_t bytes) { return bytes > kHalf; }
+    static bool fitsRow(size_t bytes) { return bytes <= kHalf; }
+    ~ReadBack() {
+        for (hipEvent_t e : filled)
+            if (e) (void)hipEventDestroy(e);
+        if (block) (void)hipHostFree(block);
+    }
+    // False when there is no page-locked memory to be had.
+    bool ready() {
+        std::lock_guard<std::mutex> lock(mutex);
+        for (hipEvent_t& e : filled)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) e = nullptr;
+        void* p = nullptr;
+        if (!block && hipHostMalloc(&p, 2 * kHalf) == hipSuccess) block = static_cast<char*>(p);
+        if (block && filled[0] && filled[1]) return true;
+        (void)hipGetLastError();
+        return false;
+    }
+    // `bytes` at `src`, after the work on `stream`, handed in pieces to
+    // take(offset, data, count).  Call ready() first, here and below.
+    template <class Take>
+    hipError_t copy(const void* src, size_t bytes, hipStream_t stream, Take&& take) {
+        auto count = [&](size_t k) { return std::min(kHalf, bytes - k * kHalf); };
+        return pump((bytes + kHalf - 1) / kHalf, stream,
+            [&](size_t k, char* half) {
+                return hipMemcpyAsync(half, static_cast<const char*>(src) + k * kHalf, count(k), hipMemcpyDeviceToHost, stream);
+            },
+            [&](size_t k, const char* half) { take(k * kHalf, half, count(k)); });
+    }
+    // Rows of rowBytes (fitsRow) `pitch` apart, side by side into `dst`.
+    hipError_t copyRows(void* dst, const void* src, size_t pitch, size_t rowBytes, size_t rows, hipStream_t stream) {
+        const size_t some = kHalf / rowBytes;
+        auto count = [&](size_t k) { return std::min(some, rows - k * some); };
+        return pump((rows + some - 1) / some, stream,
+            [&](size_t k, char* half) {
+                return hipMemcpy2DAsync(half, rowBytes, static_cast<const char*>(src) + k * some * pitch, pitch, rowBytes,
+                    count(k), hipMemcpyDeviceToHost, stream);
+            },
+            [&](size_t k, const char* half) {
+                std::memcpy(static_cast<char*>(dst) + k * some * rowBytes, half, count(k) * rowBytes);
+            });
+    }
+};
+
+// Memory that HIP knows (page-locked, managed, on a device): copies go there
+// directly.
+bool knownToHip(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
 // Triangles as queryBrute reads them.
 std::vector<float> triangleEdges(const std::vector<TriShade>& triangles) {
     std::vector<float> e;
@@ -169,6 +253,7 @@ struct wpt_renderer {
     BatchContext regen{};
     uint32_t regenBlocks = 0;
     std::vector<BatchTask> regenTasks;
+    ReadBack readBack;
     ~wpt_renderer() {
         if (stream) (void)hipStreamSynchronize(stream);
         if (exec) (void)hipGraphExecDestroy(exec);
@@ -1065,6 +1150,7 @@ WPT_API int wpt_renderer_create(wpt_scene* scene, const wpt_camera* camera, cons
         r->photonsStored = map.stored;
         if (c.caustic_gather) ctx.shade.photons = map.view;
     }
+    (void)r->readBack.ready();
     R_HIP(hipDeviceSynchronize());
 #undef R_HIP
     *out = r;
@@ -1132,7 +1218,15 @@ WPT_API int wpt_renderer_read_framebuffer(wpt_renderer* r, float* host, uint32_t
     if (!r || !host) return fail(WPT_ERROR_INVALID_ARGUMENT, "null argument");
     WPT_HIP(hipStreamSynchronize(r->stream));
     size_t n = 3 * static_cast<size_t>(r->config.width) * r->config.height;
-    WPT_HIP(hipMemcpy(host, r->ctx.framebuffer, sizeof(float) * n, hipMemcpyDeviceToHost));
+    if (ReadBack::worthwhile(sizeof(float) * n) && !knownToHip(host) && r->readBack.ready()) {
+        auto take = [&](size_t at, const char* data, size_t count) {
+            std::memcpy(reinterpret_cast<char*>(host) + at, data, count);
+        };
+        hipError_t e = r->readBack.copy(r->ctx.framebuffer, sizeof(float) * n, r->stream, take);
+        if (e != hipSuccess) return hipFail(e, "framebuffer read-back");
+    } else {
+        WPT_HIP(hipMemcpy(host, r->ctx.framebuffer, sizeof(float) * n, hipMemcpyDeviceToHost));
+    }
     if (sampleCount) {
         WavefrontCounters c;
         WPT_HIP(hipMemcpy(&c, r->ctx.counters, sizeof c, hipMemcpyDeviceToHost));
@@ -1155,8 +1249,10 @@ WPT_API int wpt_renderer_load_framebuffer(wpt_renderer* r, const float* host, ui
 WPT_API int wpt_host_alloc(uint64_t bytes, void** out) {
     if (!out || bytes == 0) return fail(WPT_ERROR_INVALID_ARGUMENT, "null output or empty block");
     *out = nullptr;
-    WPT_HIP(hipHostMalloc(out, bytes));
-    return WPT_OK;
+    hipError_t e = hipHostMalloc(out, bytes);
+    if (e == hipSuccess) return WPT_OK;
+    (void)hipGetLastError();  // no later launch failed
+    return hipFail(e, "page-locked host memory");
 }
 
 WPT_API int wpt_host_free(void* block) {
@@ -1213,8 +1309,13 @@ WPT_API int wpt_render_task(wpt_renderer* r, const wpt_task* task, float* hostTi
     r->lastSamples = static_cast<uint64_t>(task->sample_count) * task->width * task->height;
     size_t pitch = sizeof(float) * 3 * c.width;
     const float* src = r->ctx.framebuffer + (static_cast<size_t>(task->y) * c.width + task->x) * 3;
-    WPT_HIP(hipMemcpy2D(hostTile, sizeof(float) * 3 * task->width, src, pitch, sizeof(float) * 3 * task->width,
-        task->height, hipMemcpyDeviceToHost));
+    size_t row = sizeof(float) * 3 * task->width;
+    if (ReadBack::fitsRow(row) && !knownToHip(hostTile) && r->readBack.ready()) {
+        hipError_t e = r->readBack.copyRows(hostTile, src, pitch, row, task->height, r->stream);
+        if (e != hipSuccess) return hipFail(e, "tile read-back");
+    } else {
+        WPT_HIP(hipMemcpy2D(hostTile, row, src, pitch, row, task->height, hipMemcpyDeviceToHost));
+    }
     return WPT_OK;
 }
 
@@ -1344,6 +1445,7 @@ struct wpt_batch {
     uint32_t stagedCapacity = 0, stagedBlock = 0, stagedEvents = 0;
     PassPiece* pieces = nullptr;
     size_t pieceCapacity = 0;
+    ReadBack readBack;
     ~wpt_batch() {
         if (stream) (void)hipStreamSynchronize(stream);
         for (void* p : {static_cast<void*>(scenesDev), static_cast<void*>(counters), static_cast<void*>(tasks),
@@ -1864,17 +1966,28 @@ WPT_API int wpt_batch_render(wpt_batch* b, const wpt_batch_task* tasks, uint32_t
     }
     b->last.samples = samples;
     b->last.milliseconds = ms;
-    size_t total = 0;
-    bool contiguous = true;  // the outputs lie side by side, as on the device
-    for (uint32_t i = 0; i < n; ++i) {
-        contiguous = contiguous && outs[i] == outs[0] + total;
-        total += 3ull * tasks[i].tile_width * tasks[i].tile_height;
+    auto bytesOf = [&](uint32_t i) -> size_t { return sizeof(float) * 3ull * tasks[i].tile_width * tasks[i].tile_height; };
+    if (n && !knownToHip(outs[0]) && b->readBack.ready()) {  // the outputs lie side by side on the device
+        uint32_t task = 0;
+        size_t done = 0;  // bytes of the task's output written
+        auto take = [&](size_t, const char* data, size_t count) {
+            while (count) {
+                size_t part = std::min(count, bytesOf(task) - done);
+                std::memcpy(reinterpret_cast<char*>(outs[task]) + done, data, part);
+                data += part;
+                count -= part;
+                done += part;
+                if (done < bytesOf(task)) break;
+                ++task;
+                done = 0;
+            }
+        };
+        hipError_t e = b->readBack.copy(b->out, sizeof(float) * offsets[n - 1] + bytesOf(n - 1), b->stream, take);
+        if (e != hipSuccess) return hipFail(e, "batch read-back");
+    } else {
+        for (uint32_t i = 0; i < n; ++i)
+            WPT_HIP(hipMemcpy(outs[i], b->out + offsets[i], bytesOf(i), hipMemcpyDeviceToHost));
     }
-    std::vector<float> host(contiguous ? 0 : total);
-    float* copied = contiguous && n ? outs[0] : host.data();
-    if (total) WPT_HIP(hipMemcpy(copied, b->out, sizeof(float) * total, hipMemcpyDeviceToHost));
-    for (uint32_t i = 0; i < n && !contiguous; ++i)
-        std::memcpy(outs[i], host.data() + offsets[i], sizeof(float) * 3ull * tasks[i].tile_width * tasks[i].tile_height);
     if (latencyMs && n && !staged) {
         std::vector<BatchTaskState> state(n);
         WPT_HIP(hipMemcpy(state.data(), b->state, sizeof(BatchTaskState) * n, hipMemcpyDeviceToHost));

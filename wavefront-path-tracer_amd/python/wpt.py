@@ -10,8 +10,6 @@ from __future__ import annotations
 
 import ctypes as C
 import os
-import threading
-import weakref
 from typing import Iterable, List, Optional, Sequence
 
 import numpy as np
@@ -694,71 +692,6 @@ def render_config(width, height, spp=1, max_depth=8, rr_start=3, block_size=256,
     return rc
 
 
-class _Block:
-    """A page-locked block as numpy sees it; arrays over it keep it alive."""
-
-    def __init__(self, address: int, floats: int):
-        self.__array_interface__ = {"data": (address, False), "shape": (floats,), "typestr": "<f4", "version": 3}
-
-
-class _ResultBlocks:
-    """Page-locked blocks that results are read back into, of one renderer or
-    batch.  An array's block comes back when the last array over it is gone;
-    KEPT free blocks are kept until the owner is closed, at most LIVE are
-    handed out at a time (results beyond that, or larger than LARGEST, get
-    ordinary memory).  A 1080p framebuffer is read in 0.5 ms so, in 1.8 ms
-    into new pageable memory."""
-    KEPT, LIVE, LARGEST = 2, 4, 1 << 28
-
-    def __init__(self):
-        self._lock = threading.RLock()  # a collected array may give its block back in here
-        self._free = []  # (address, bytes)
-        self._live = 0
-        self._closed = False
-
-    def _take(self, size: int):
-        with self._lock:
-            if size == 0 or size > self.LARGEST or self._live >= self.LIVE or self._closed:
-                return None
-            self._live += 1
-            for k, (address, have) in enumerate(self._free):
-                if have >= size:
-                    return self._free.pop(k)
-            stale = self._free.pop(0) if len(self._free) >= self.KEPT else None
-        if stale:
-            library().wpt_host_free(stale[0])
-        address = C.c_void_p()
-        if library().wpt_host_alloc(size, C.byref(address)) != OK:
-            with self._lock:
-                self._live -= 1
-            return None
-        return address.value, size
-
-    def _give(self, address: int, size: int):
-        with self._lock:
-            self._live -= 1
-            if not self._closed and len(self._free) < self.KEPT:
-                self._free.append((address, size))
-                return
-        library().wpt_host_free(address)
-
-    def array(self, shape) -> np.ndarray:
-        floats = int(np.prod(shape, dtype=np.int64))
-        block = self._take(4 * floats)
-        if block is None:
-            return np.empty(shape, np.float32)
-        owner = _Block(block[0], floats)
-        weakref.finalize(owner, self._give, *block).atexit = False
-        return np.asarray(owner).reshape(shape)
-
-    def close(self):
-        with self._lock:
-            self._closed = True
-            free, self._free = self._free, []
-        for address, _ in free:
-            library().wpt_host_free(address)
-
-
 class Renderer:
     def __init__(self, scene: Scene, camera: Camera, config: RenderConfig, fingerprint: int = 0):
         self.scene, self.camera, self.config = scene, camera, config
@@ -766,9 +699,6 @@ class Renderer:
         self._h = C.c_void_p()
         check(library().wpt_renderer_create(scene.handle, C.byref(camera), C.byref(config), fingerprint,
                                             C.byref(self._h)), "wpt_renderer_create")
-        self._blocks = _ResultBlocks()
-        # The first frame's block, with the renderer's other buffers.
-        self._blocks.array((config.height, config.width, 3))
 
     def reset(self):
         check(library().wpt_renderer_reset(self._h), "wpt_renderer_reset")
@@ -778,7 +708,7 @@ class Renderer:
 
     def framebuffer(self):
         c = self.config
-        out = self._blocks.array((c.height, c.width, 3))
+        out = np.empty((c.height, c.width, 3), np.float32)
         n = C.c_uint32()
         check(library().wpt_renderer_read_framebuffer(self._h, out.ctypes.data, C.byref(n)),
               "wpt_renderer_read_framebuffer")
@@ -792,13 +722,13 @@ class Renderer:
 
     def render_frame(self):
         c = self.config
-        out = self._blocks.array((c.height, c.width, 3))
+        out = np.empty((c.height, c.width, 3), np.float32)
         n = C.c_uint32()
         check(library().wpt_render_frame(self._h, out.ctypes.data, C.byref(n)), "wpt_render_frame")
         return out, n.value
 
     def render_task(self, task: Task):
-        out = self._blocks.array((task.height, task.width, 3))
+        out = np.empty((task.height, task.width, 3), np.float32)
         check(library().wpt_render_task(self._h, C.byref(task), out.ctypes.data), "wpt_render_task")
         return out
 
@@ -825,7 +755,6 @@ class Renderer:
         if self._h:
             library().wpt_renderer_destroy(self._h)
             self._h = C.c_void_p()
-            self._blocks.close()
 
     def __del__(self):
         try:
@@ -853,7 +782,6 @@ class Batch:
         cfg = BatchConfig(block_size, blocks, scheduler, pass_paths)
         check(library().wpt_batch_create(handles, len(self._scenes), C.byref(cfg), C.byref(self._h)),
               "wpt_batch_create")
-        self._blocks = _ResultBlocks()
 
     def set_caustics(self, scene_index: int, config: RenderConfig):
         """Builds scene `scene_index`'s caustic photon map from the caustic
@@ -873,10 +801,7 @@ class Batch:
         """Returns a list of (tile_height, tile_width, 3) float32 sums, and the
         per-task latencies in ms when asked."""
         arr = self._tasks(tasks)
-        sizes = [3 * t.tile_height * t.tile_width for t in tasks]
-        whole = self._blocks.array((sum(sizes),))  # the outputs side by side, read back in one copy
-        starts = np.cumsum([0] + sizes)
-        outs = [whole[a:a + n].reshape(t.tile_height, t.tile_width, 3) for a, n, t in zip(starts, sizes, tasks)]
+        outs = [np.empty((t.tile_height, t.tile_width, 3), np.float32) for t in tasks]
         ptrs = (C.c_void_p * max(1, len(tasks)))(*[o.ctypes.data for o in outs])
         lat = np.zeros(max(1, len(tasks)), np.float64)
         check(library().wpt_batch_render(self._h, arr, len(tasks), ptrs, lat.ctypes.data if latencies else None),
@@ -898,7 +823,6 @@ class Batch:
         if self._h:
             library().wpt_batch_destroy(self._h)
             self._h = C.c_void_p()
-            self._blocks.close()
 
     def __del__(self):
         try:
