@@ -145,3 +145,18 @@ def test_rays_at_edges_of_flat_trees(torch_cuda, oracle_mod, accel, bump):
     assert np.allclose(got["t"], want["t"], rtol=1e-3)
     for p, q in zip(*(h["primitive"][got["primitive"] != want["primitive"]] for h in (got, want))):
         assert len(set(map(tuple, verts[p])) & set(map(tuple, verts[q]))) > 0, (p, q)
+
+
+def test_spill_columns_are_sized_to_the_scene(torch_cuda):
+    """A scene of twelve triangles has no deep walks: a regenerating renderer,
+    which has no path queues, takes a frame and little else, where 80 stack
+    entries for each of its threads alone would be 1 GB."""
+    host = wpt.HostScene("cornell-box")
+    scene = wpt.Scene(host.desc(), device=True, owner=host)
+    torch_cuda.cuda.synchronize()
+    before = torch_cuda.cuda.mem_get_info()[0]
+    r = wpt.Renderer(scene, host.camera(1920, 1080),
+                     wpt.render_config(1920, 1080, spp=1, max_depth=4, mode=wpt.MODE_REGENERATE))
+    used = before - torch_cuda.cuda.mem_get_info()[0]
+    r.close()
+    assert used < 1 << 28, used

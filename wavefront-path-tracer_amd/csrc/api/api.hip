@@ -716,7 +716,7 @@ WPT_API int wpt_scene_export_light_indices(const wpt_scene* s, uint32_t* instanc
 static int ensureAbiSpill(wpt_scene* s) {
     if (s->abiSpill) return WPT_OK;
     void* p = nullptr;
-    size_t bytes = sizeof(uint2) * (kMaxStackDepth - kLdsStackEntries) * static_cast<size_t>(abiTraceThreads());
+    size_t bytes = sizeof(uint2) * spillEntries(walkStackEntries(s->host)) * static_cast<size_t>(abiTraceThreads());
     WPT_HIP(s->arena.alloc(bytes, &p));
     s->abiSpill = static_cast<uint2*>(p);
     return WPT_OK;
@@ -1138,7 +1138,7 @@ WPT_API int wpt_renderer_create(wpt_scene* scene, const wpt_camera* camera, cons
     }
     // One spill column per thread index of any grid.
     ctx.spillThreads = std::max(std::max(ctx.gridBlocks, ctx.persistentBlocks), r->regenBlocks) * c.block_size;
-    R_HIP(r->arena.alloc(sizeof(uint2) * (kMaxStackDepth - kLdsStackEntries) * static_cast<size_t>(ctx.spillThreads), &p));
+    R_HIP(r->arena.alloc(sizeof(uint2) * spillEntries(walkStackEntries(scene->host)) * static_cast<size_t>(ctx.spillThreads), &p));
     ctx.spill = static_cast<uint2*>(p);
     r->regen.spill = ctx.spill;
     r->regen.spillThreads = ctx.spillThreads;
@@ -1552,13 +1552,20 @@ int stageBatch(wpt_batch* b, const wpt_batch_task* tasks, uint32_t n, std::vecto
     return WPT_OK;
 }
 
+// Of the deepest of the batch's scenes, which share the columns.
+uint32_t batchSpillEntries(const wpt_batch* b) {
+    uint32_t entries = 0;
+    for (const wpt_scene* s : b->scenes) entries = std::max(entries, walkStackEntries(s->host));
+    return spillEntries(entries);
+}
+
 // Traversal spill columns for `threads` threads.
 int ensureBatchSpill(wpt_batch* b, uint32_t threads) {
     if (threads <= b->spillThreads) return WPT_OK;
     if (b->spill) WPT_HIP(hipFree(b->spill));
     b->spill = nullptr;
     b->spillThreads = 0;
-    WPT_HIP(hipMalloc(reinterpret_cast<void**>(&b->spill), sizeof(uint2) * kSpillEntriesTotal * static_cast<size_t>(threads)));
+    WPT_HIP(hipMalloc(reinterpret_cast<void**>(&b->spill), sizeof(uint2) * batchSpillEntries(b) * static_cast<size_t>(threads)));
     b->spillThreads = threads;
     return WPT_OK;
 }
@@ -1696,7 +1703,7 @@ int ensureStagedBatch(wpt_batch* b, uint32_t blockSize, uint32_t paths) {
     ctx.counters = static_cast<WavefrontCounters*>(p);
     WPT_HIP(hipMemset(p, 0, sizeof(WavefrontCounters)));
     ctx.spillThreads = ctx.gridBlocks * B;
-    WPT_HIP(arena.alloc(sizeof(uint2) * kSpillEntriesTotal * static_cast<size_t>(ctx.spillThreads), &p));
+    WPT_HIP(arena.alloc(sizeof(uint2) * batchSpillEntries(b) * static_cast<size_t>(ctx.spillThreads), &p));
     ctx.spill = static_cast<uint2*>(p);
     ctx.profileQueues = 0;
     ctx.slots = 1;
@@ -2170,7 +2177,7 @@ WPT_API int wpt_diff_create(wpt_scene* scene, const wpt_camera* camera, const wp
     d->forwardBlocks = static_cast<uint32_t>(std::min<uint64_t>(pathBlocks, static_cast<uint64_t>(forwardPerCu) * cus));
     d->adjointBlocks = static_cast<uint32_t>(std::min<uint64_t>(pathBlocks, static_cast<uint64_t>(adjointPerCu) * cus));
     x.spillThreads = std::max(d->forwardBlocks, d->adjointBlocks) * c.block_size;
-    D_HIP(d->arena.alloc(sizeof(uint2) * kSpillEntriesTotal * static_cast<size_t>(x.spillThreads), &mem));
+    D_HIP(d->arena.alloc(sizeof(uint2) * spillEntries(walkStackEntries(scene->host)) * static_cast<size_t>(x.spillThreads), &mem));
     x.spill = static_cast<uint2*>(mem);
 #undef D_HIP
     d->stats.paths = paths;

@@ -314,63 +314,10 @@ __global__ void __launch_bounds__(kBlock) kLeafDepth(const uint32_t* leafParent,
     if (threadIdx.x == 0) atomicMax(depth, best[0]);
 }
 
-// Quad node i from binary node i: its two children, each opened into its own
-// two if it is interior, then the largest interior child opened until there
-// are four.  One thread per node; a scene's upload runs it once per tree.
+// One thread per node; a scene's upload runs it once per tree.
 __global__ void __launch_bounds__(kBlock) kCollapseQuads(const BvhNode* nodes, uint32_t count, QuadNode* out) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    float box[kQuadChildren][6];
-    uint32_t child[kQuadChildren];
-    auto open = [&](uint32_t node, uint32_t left, uint32_t right) {
-        const BvhNode n = nodes[node];
-        const float l[6] = {n.lminx, n.lminy, n.lminz, n.lmaxx, n.lmaxy, n.lmaxz};
-        const float r[6] = {n.rminx, n.rminy, n.rminz, n.rmaxx, n.rmaxy, n.rmaxz};
-        for (int k = 0; k < 6; ++k) {
-            box[left][k] = l[k];
-            box[right][k] = r[k];
-        }
-        child[left] = n.left;
-        child[right] = n.right;
-    };
-    open(i, 0u, 1u);
-    uint32_t used = 2u;
-    const bool openLeft = !(child[0] & kLeafBit), openRight = !(child[1] & kLeafBit);
-    if (openLeft) open(child[0], 0u, used++);
-    if (openRight) open(child[1], 1u, used++);
-    while (used < kQuadChildren) {
-        uint32_t best = kInvalid;
-        float area = -1.0f;
-        for (uint32_t k = 0; k < used; ++k) {
-            if (child[k] & kLeafBit) continue;
-            float dx = box[k][3] - box[k][0], dy = box[k][4] - box[k][1], dz = box[k][5] - box[k][2];
-            float a = dx * dy + dy * dz + dz * dx;
-            if (best == kInvalid || a > area) {
-                best = k;
-                area = a;
-            }
-        }
-        if (best == kInvalid) break;
-        open(child[best], best, used++);
-    }
-    const float inf = __builtin_inff();
-    for (uint32_t k = used; k < kQuadChildren; ++k) {
-        child[k] = kInvalid;
-        for (int c = 0; c < 3; ++c) {
-            box[k][c] = inf;
-            box[k][3 + c] = -inf;
-        }
-    }
-    QuadNode q;
-    for (uint32_t k = 0; k < kQuadChildren; ++k) {
-        for (int c = 0; c < 3; ++c) {
-            q.mn[c][k] = box[k][c];
-            q.mx[c][k] = box[k][3 + c];
-        }
-        q.child[k] = child[k];
-        q.pad[k] = 0u;
-    }
-    out[i] = q;
+    if (i < count) out[i] = quadNode(nodes, i);
 }
 
 // Device allocations of one build, released on every exit.

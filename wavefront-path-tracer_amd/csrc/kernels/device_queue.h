@@ -9,8 +9,6 @@
 
 namespace wpt {
 
-constexpr uint32_t kSpillEntries = kMaxStackDepth - kLdsStackEntries;
-
 // Occupancy target of the traversal kernels (waves per SIMD), 0: compiler's
 // choice.  The register budget it implies must not force scratch spills.
 // The batch kernel has its own targets with (Full) and without the full

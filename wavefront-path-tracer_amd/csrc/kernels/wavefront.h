@@ -109,7 +109,11 @@ struct WavefrontCounters {
 #define WPT_LDS_STACK_ENTRIES 16
 #endif
 constexpr uint32_t kLdsStackEntries = WPT_LDS_STACK_ENTRIES;
-constexpr uint32_t kSpillEntriesTotal = kMaxStackDepth - kLdsStackEntries;  // per thread
+// Entries of a spill column for walks that hold at most `entries`
+// (walkStackEntries): a scene pays for its own trees' depth on every thread.
+inline uint32_t spillEntries(uint32_t entries) {
+    return entries > kLdsStackEntries ? entries - kLdsStackEntries : 1u;
+}
 
 struct LaunchContext {
     DevScene scene;
@@ -140,7 +144,7 @@ struct LaunchContext {
     uint32_t width, height;
     WavefrontCounters* counters;
     const RenderTile* tile;  // device copy of the current tile
-    uint2* spill;            // (kMaxStackDepth - kLdsStackEntries) x spillThreads, one column per thread index
+    uint2* spill;            // spillEntries x spillThreads, one column per thread index
     uint32_t spillThreads;
     uint32_t capacity;         // tile pixels x slots: the most items any queue holds
     uint32_t blockSize;
@@ -291,7 +295,7 @@ hipError_t batchAttributes(bool full, hipFuncAttributes* out);
 hipError_t kernelAttributes(bool persistent, bool full, hipFuncAttributes* out, bool events = true);
 
 // Standalone traversal for the C ABI; `spill` holds
-// (kMaxStackDepth - kLdsStackEntries) x abiTraceThreads() entries.
+// spillEntries x abiTraceThreads() entries.
 uint32_t abiTraceThreads();
 hipError_t launchTraceClosest(const DevScene& scene, const float* rays6, uint32_t n, void* hitsOut, uint2* spill,
     hipStream_t stream);

@@ -372,6 +372,13 @@ uint32_t stackDepth(const HostSceneData& s) {
     return std::max(s.tlas.depth + s.maxBlasDepth + 2, flat);
 }
 
+uint32_t walkStackEntries(const HostSceneData& s) {
+    // Per four-wide level three entries; a level spans at least two binary ones.
+    auto quads = [](uint32_t depth) { return 3u * ((depth + 1u) / 2u); };
+    uint32_t flat = s.flatWide.empty() ? quads(s.flat.depth) : s.flatWideStack;
+    return std::max(quads(s.tlas.depth) + quads(s.maxBlasDepth), flat);
+}
+
 HostBvh buildBvh2(const std::vector<Aabb>& primBounds, unsigned threads, bool median) {
     HostBvh bvh;
     bvh.primBounds = primBounds;

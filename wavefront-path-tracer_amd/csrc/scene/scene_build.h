@@ -123,4 +123,8 @@ std::string buildHostScene(const wpt_scene_desc& desc, HostSceneData& out, unsig
 // the flat BVH.
 uint32_t stackDepth(const HostSceneData& s);
 
+// Most traversal-stack entries that a kernel's walk of the scene holds at a
+// time: of the TLAS and the deepest BLAS together, or of the flat tree.
+uint32_t walkStackEntries(const HostSceneData& s);
+
 }  // namespace wpt
