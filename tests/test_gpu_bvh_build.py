@@ -158,3 +158,23 @@ def test_device_builder_needs_a_device_scene():
         wpt.Scene(with_builder(b.desc(), wpt.BVH_DEVICE_PLOC), device=False, owner=b)
     with pytest.raises(wpt.WptError):
         wpt.Scene(with_builder(b.desc(), wpt.BVH_DEVICE_PLOC, 65), device=True, owner=b)
+
+
+def test_device_built_scene_keeps_no_binary_nodes(torch_cuda):
+    # Host- and device-built scenes hold the same arrays: the binary tree is
+    # gone after the four-wide nodes are made of it, and an export of it later
+    # leaves nothing behind.
+    host = wpt.HostScene("sphere-field")
+
+    def taken(builder):
+        torch_cuda.cuda.synchronize()
+        before = torch_cuda.cuda.mem_get_info()[0]
+        scene = wpt.Scene(with_builder(host.desc(), builder), device=True, owner=host)
+        scene.export_bvh2(2)
+        used = before - torch_cuda.cuda.mem_get_info()[0]
+        scene.close()
+        return used
+
+    taken(wpt.BVH_DEVICE_PLOC)  # the builder's code and scratch
+    sah, ploc = taken(wpt.BVH_HOST_SAH), taken(wpt.BVH_DEVICE_PLOC)
+    assert sah > 100 << 20 and abs(ploc - sah) < 16 << 20, (sah, ploc)

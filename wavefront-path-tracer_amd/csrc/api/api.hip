@@ -213,10 +213,10 @@ Bvh deviceBvhView(const HostBvh& h, const QuadNode* nodes) {
 
 }  // namespace
 
-// A BLAS built on the device: where its nodes and slot order live.
+// A BLAS built on the device.  Its binary nodes and slot order go once the
+// quad nodes are made (68 of 196 B a triangle); an export builds them again.
 struct DeviceBlas {
-    const BvhNode* nodes = nullptr;
-    const uint32_t* order = nullptr;
+    const TriShade* triangles = nullptr;
     uint32_t primCount = 0;
     DeviceBvhBuild build{};
 };
@@ -469,11 +469,12 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
             if (mesh.buildOnDevice && status == WPT_OK) {
                 // Device construction straight into the scene's arena.
                 uint32_t n = b.triangleCount;
+                DeviceArena binary;
                 void *nodes = nullptr, *quads = nullptr, *geometry = nullptr, *order = nullptr;
-                check(a.alloc(sizeof(BvhNode) * (n - 1), &nodes), "blas nodes");
+                check(binary.alloc(sizeof(BvhNode) * (n - 1), &nodes), "blas nodes");
                 check(a.alloc(sizeof(QuadNode) * (n - 1), &quads), "blas quad nodes");
                 check(a.alloc(sizeof(float4) * 3 * static_cast<size_t>(n), &geometry), "blas geometry");
-                check(a.alloc(sizeof(uint32_t) * n, &order), "blas order");
+                check(binary.alloc(sizeof(uint32_t) * n, &order), "blas order");
                 DeviceBlas& rec = s->deviceBlas[m];
                 if (status == WPT_OK)
                     check(buildTriangleBvh(b.triangles, n, h.bvhSearchRadius, static_cast<BvhNode*>(nodes),
@@ -482,8 +483,8 @@ static int createScene(const wpt_scene_desc* desc, wpt_scene** out, bool upload)
                 if (status == WPT_OK)
                     check(collapseQuads(static_cast<const BvhNode*>(nodes), n - 1, static_cast<QuadNode*>(quads), nullptr),
                         "quad nodes");
-                rec.nodes = static_cast<const BvhNode*>(nodes);
-                rec.order = static_cast<const uint32_t*>(order);
+                check(hipStreamSynchronize(nullptr), "quad nodes");  // before the binary nodes go
+                rec.triangles = b.triangles;
                 rec.primCount = n;
                 b.bvh = Bvh{};
                 b.bvh.nodes = static_cast<const QuadNode*>(quads);
@@ -631,16 +632,25 @@ WPT_API int wpt_scene_export_bvh2(const wpt_scene* s, uint32_t bvh, wpt_bvh2_nod
     else if (bvh - 2 < s->host.meshes.size()) h = &s->host.meshes[bvh - 2].bvh;
     else return fail(WPT_ERROR_INVALID_ARGUMENT, "unknown BVH");
     if (bvh >= 2 && s->deviceBlas[bvh - 2].primCount) {
-        // A device-built BLAS: nodes and slot order back from the device,
-        // leaf bounds recomputed from the triangles as the builder did.
+        // A device-built BLAS: nodes and slot order built once more (repeated
+        // builds are identical) and back from the device, leaf bounds
+        // recomputed from the triangles as the builder did.
         const DeviceBlas& d = s->deviceBlas[bvh - 2];
         const HostMesh& mesh = s->host.meshes[bvh - 2];
+        DeviceArena binary;
+        void *nodes = nullptr, *geometry = nullptr, *order = nullptr;
+        WPT_HIP(binary.alloc(sizeof(BvhNode) * (d.primCount - 1), &nodes));
+        WPT_HIP(binary.alloc(sizeof(float4) * 3 * static_cast<size_t>(d.primCount), &geometry));
+        WPT_HIP(binary.alloc(sizeof(uint32_t) * d.primCount, &order));
+        DeviceBvhBuild again{};
+        WPT_HIP(buildTriangleBvh(d.triangles, d.primCount, s->host.bvhSearchRadius, static_cast<BvhNode*>(nodes),
+            static_cast<float4*>(geometry), static_cast<uint32_t*>(order), nullptr, &again));
         fetched.nodes.resize(d.primCount - 1);
         fetched.order.resize(d.primCount);
         if (d.primCount > 1)
-            WPT_HIP(hipMemcpy(fetched.nodes.data(), d.nodes, sizeof(BvhNode) * (d.primCount - 1),
+            WPT_HIP(hipMemcpy(fetched.nodes.data(), nodes, sizeof(BvhNode) * (d.primCount - 1),
                 hipMemcpyDeviceToHost));
-        WPT_HIP(hipMemcpy(fetched.order.data(), d.order, sizeof(uint32_t) * d.primCount, hipMemcpyDeviceToHost));
+        WPT_HIP(hipMemcpy(fetched.order.data(), order, sizeof(uint32_t) * d.primCount, hipMemcpyDeviceToHost));
         for (const TriShade& t : mesh.triangles) fetched.primBounds.push_back(triangleBounds(t.v0, t.v1, t.v2));
         fetched.root = d.primCount > 1 ? 0u : (kLeafBit | 0u);
         fetched.depth = d.build.depth;
