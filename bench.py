@@ -9,18 +9,19 @@ geodesic icosphere of 1,003,520 triangles.  1920x1080, 64 spp, depth 12,
 Russian roulette from depth 3, PCG32 streams, indirect clamp 10.
 
 One step = one full frame (64 spp) rendered into the device framebuffer by
-the chosen scheduler (default: the persistent kernel with path
-regeneration); the scene is resident in HBM before the timed region.
+the chosen scheduler (default: the hipGraph-captured staged wavefront); the
+scene is resident in HBM before the timed region.
 `value` is Mrays/s = (closest-hit + shadow queries) / s; Msamples/s and the
-rates of the other two schedulers (hipGraph-captured staged wavefront,
+rates of the other two schedulers (the kernel with path regeneration, the
 cooperative persistent kernel), with a check that their images are
 identical, are reported beside it.
 
-The roofline object is for the dominant kernel (the regenerating kernel, or
-the closest-hit trace of the staged wavefront), timed with HIP events on the
-renderer's stream; its algorithmic bytes per query follow the reference
-algorithm's work counts (node tests, triangle/sphere tests, instance
-entries) measured by the CPU oracle on the same scene and BVH.
+The roofline object is for the dominant kernel (the closest-hit trace of the
+staged wavefront, or the regenerating kernel), timed with HIP events on the
+renderer's stream.  What bounds it is VALU issue, by the profiler's counters;
+the HBM rate comes from measured traffic, and the rate in the reference's data
+model from its work counts (node tests, triangle/sphere tests, instance
+entries), measured by the CPU oracle on the same scene and BVH.
 The CPU baseline is the oracle (the scalar FP32 restatement of the reference
 traversal and shading) on the host cores, over a bounded sample.
 
@@ -45,24 +46,34 @@ import wpt  # noqa: E402
 METRIC = "Mrays/s + Msamples/s at 1080p 64spp; batched vs plain; fwd+adjoint ms/iter"
 WIDTH, HEIGHT, SPP, DEPTH, RR_START, CLAMP = 1920, 1080, 64, 12, 3, 10.0
 HBM_PEAK_GBS = 8000.0
-# Bytes per unit of work in the reference algorithm's data model: a BVH node
-# record (AABB + two child words), a triangle's three vertices, a sphere
-# (center, radius, material), a mesh-instance record (transforms + ids).
+# Bytes per unit of work in the reference algorithm's data model: a binary BVH
+# node record (AABB + two child words), a triangle's three vertices, a sphere
+# (center, radius, material), a mesh-instance record (transforms + ids).  The
+# kernels walk four-wide nodes of 128 B and visit fewer of them, so these bytes
+# over a kernel's time are a rate of work, not of memory.
 NODE_B, TRI_B, SPHERE_B, INSTANCE_B = 32, 36, 20, 96
 RAY_IN_B, HIT_OUT_B = 24, 28
 # HBM bytes per launch of the dominant kernel on this workload, from
 # rocprofv3 FETCH_SIZE / WRITE_SIZE runs scaled by a 256 MiB copy kernel
 # (FETCH_SIZE reads 131086 KiB for it: x2.000; WRITE_SIZE 262144 KiB: x1.000),
 # with the counters that say what bounds it.  kTrace: average of the 12
-# launches (bounces) of one 64-sample pass of the staged scheduler
-# (profiles/pmc_kTrace_sphere_field_1080p_64spp.md); kBatch: one 64-sample
+# launches (bounces) of one 64-sample pass of the staged scheduler, the camera
+# bounce's kTracePrimary among them; the counters are those of the other 11
+# (profiles/pmc_kTrace_sphere_field_1080p_64spp.md).  kBatch: one 64-sample
 # frame of the regenerating scheduler
 # (profiles/pmc_kBatch_sphere_field_1080p_64spp.md).
-MEASURED_TRAFFIC = {("kTrace", 64): 46.84e9 / 12, ("kBatch", 64): 39.21e9}
+MEASURED_TRAFFIC = {("kTrace", 64): 35.07e9 / 12, ("kBatch", 64): 29.83e9}
 MEASURED_COUNTERS = {
-    ("kTrace", 64): {"l2_hit": 0.515, "valu_busy": 0.757, "waves_per_cu": 12.14, "wait_any": 0.526,
-                     "lanes_active": 0.257, "l1_hit": 0.904, "ta_busy": 0.485, "l1_to_l2_latency_cycles": 306},
-    ("kBatch", 64): {"l2_hit": 0.615, "valu_busy": 0.303, "waves_per_cu": 7.87, "wait_any": 0.672},
+    ("kTrace", 64): {"l2_hit": 0.477, "valu_busy": 0.956, "waves_per_cu": 12.12, "wait_any": 0.464,
+                     "lanes_active": 0.331, "l1_hit": 0.921, "ta_busy": 0.522, "l1_to_l2_latency_cycles": 322},
+    ("kBatch", 64): {"l2_hit": 0.596, "valu_busy": 0.459, "waves_per_cu": 8.89, "wait_any": 0.635,
+                     "lanes_active": 0.213},
+}
+LIMITERS = {
+    "kTrace": "VALU issue: busy 96% of the time with a third of the lanes active (turns of one visit kind per wave); "
+              "HBM carries a ninth of its peak",
+    "kBatch": "chains of dependent node fetches at 3 waves per SIMD, with a fifth of the lanes of a VALU instruction "
+              "active where shading and shadow rays take turns",
 }
 
 
@@ -872,21 +883,22 @@ def main():
             # One kernel does every query; paths stay in registers.
             per_query = closest_b
             algorithmic = closest_b * prof_closest + shadow_b * prof_shadow
-        achieved = algorithmic / (trace_ms / 1000.0) / 1e9
         kernel = {wpt.MODE_GRAPH: "kTrace", wpt.MODE_PERSISTENT: "kPersistent", wpt.MODE_REGENERATE: "kBatch"}[mode]
+        traffic = MEASURED_TRAFFIC.get((kernel, args.spp))
+        valu = (MEASURED_COUNTERS.get((kernel, args.spp)) or {}).get("valu_busy")
+        hbm = traffic / (trace_ms / max(1, trace_launches) / 1000.0) / 1e9 if traffic else None
         roofline = {
-            "bound": "hbm",
-            "achieved": round(achieved, 1),
-            "peak": HBM_PEAK_GBS,
-            "unit": "GB/s",
-            "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "bound": "valu issue",
+            "achieved": valu,
+            "peak": 1.0,
+            "unit": "share of issue cycles",
+            "frac": valu,
             "kernel": kernel,
-            "traffic": MEASURED_TRAFFIC.get((kernel, args.spp)),
-            "hbm_gbs_measured": None if (kernel, args.spp) not in MEASURED_TRAFFIC else
-                round(MEASURED_TRAFFIC[(kernel, args.spp)] / (trace_ms / max(1, trace_launches) / 1000.0) / 1e9, 1),
-            "limiter": "chains of dependent node and triangle fetches (L1 serves 90%, L2 half of the rest at "
-                       "306 cycles) with a quarter of the lanes active: VALU busy 76%, the address path half busy; "
-                       "the algorithmic bytes count every node visit and the measured HBM traffic is a small part",
+            "traffic": traffic,
+            "hbm_gbs_measured": hbm and round(hbm, 1),
+            "hbm_frac": hbm and round(hbm / HBM_PEAK_GBS, 4),
+            "reference_model_gbs": round(algorithmic / (trace_ms / 1000.0) / 1e9, 1),
+            "limiter": LIMITERS.get(kernel),
             "counters": MEASURED_COUNTERS.get((kernel, args.spp)),
             "bytes_per_closest_query": round(per_query, 1),
             "avg_launch_ms": round(trace_ms / max(1, trace_launches), 4),
