@@ -490,12 +490,13 @@ WPT_API int wpt_render_task(wpt_renderer* renderer, const wpt_task* task, float*
 WPT_API int wpt_renderer_last_stats(const wpt_renderer* renderer, wpt_stats* stats);
 /* Renders samples [first, first+count) with every kernel launch bracketed by
  * HIP events on the renderer's stream (no graph), accumulating device time
- * per kernel into kernel_ms[7] and launch counts into launches[7]: 0 primary
- * rays, 1 queue reset with the kernel that ends small queues' paths, 2
- * closest-hit trace, 3 shade, 4 persistent, 5 shadow rays (with radiance
- * events: the event rays and the pass adding the
- * unblocked contributions), 6 pass resolve (a pass's samples added to the
- * framebuffer in sample order). */
+ * per kernel into kernel_ms[7] and launch counts into launches[7]: 0 start of
+ * a pass (passes of at most 131072 paths: the primary rays; larger ones make
+ * them in slots 2 and 3), 1 queue reset with the kernel that ends small queues'
+ * paths, 2 closest-hit trace, 3 shade, 4 persistent, 5 shadow rays (with
+ * radiance events: the event rays and the pass adding the unblocked
+ * contributions), 6 pass resolve (a pass's samples added to the framebuffer in
+ * sample order). */
 WPT_API int wpt_renderer_profile_kernels(wpt_renderer* renderer, uint32_t first_sample, uint32_t count,
                                          double* kernel_ms, uint32_t* launches);
 

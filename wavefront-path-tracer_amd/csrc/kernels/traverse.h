@@ -183,7 +183,7 @@ WPT_HD bool slab(const RayInv& r, float mnx, float mny, float mnz, float mxx, fl
 // still depend on the order of visits, where a triangle is hit a little before
 // the ray enters its box (rounding at an edge) and the other's distance lies
 // between: of rays aimed at edges 1 in 1e5 (overlapping boxes of a median tree)
-// to less than 1 in 1e7 (SAH) hit the neighbour that a binary walk does not.
+// to about 1 in 1e7 (SAH) hit the neighbour that a binary walk does not.
 // Rays with a component outside 2^-60 .. 2^60 in size (a zero component of the
 // direction has an infinite inverse), which would overflow, take slab() at
 // every node: their nearBias.x is NaN.
@@ -399,8 +399,8 @@ WPT_HD bool queryBvh(const DevScene& s, const RayInv& r, const Bvh& bvh, const f
     while (true) {
         if (cur & kLeafBit) {
             uint32_t slot = cur & ~kLeafBit;
-            // A clipped leaf's box first: held through the triangle's test it
-            // costs kTrace five spills (terrain 4% slower).
+            // A clipped leaf's box first: fetched after the triangle's test it
+            // costs kTrace five spills (terrain 1080p, 16 spp: 136.4 -> 139.0 ms).
             if (!s.flatClipped || slotOpen(geometry + 3 * bvh.primCount, r, slot, best.t)) {
                 float4 a = geometry[3 * slot + 0];
                 float4 e = geometry[3 * slot + 1];

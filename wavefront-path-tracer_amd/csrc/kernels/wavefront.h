@@ -157,8 +157,10 @@ struct LaunchContext {
 
 // Queues that kTail takes over (LaunchContext.tailPaths): above it a bounce's
 // rays keep the chip busy for longer than its longest walk (sphere field and
-// Cornell box frames and batches: 32768 up to 16% slower, 524288 up to 22%),
-// and the lanes of its grid, what is resident at three waves per SIMD.
+// Cornell box frames and batches: 32768 up to 16% slower, 524288 up to 22%;
+// radiance events, terrain 480x270 with 8 samples: 12.2 / 12.0 / 12.0 / 15.7 ms
+// at 32768 / 65536 / 131072 / 262144, 1080p with 16: 137.9 / 137.6 / 136.4 /
+// 140.5), and the lanes of its grid, what is resident at three waves per SIMD.
 constexpr uint32_t kTailPaths = 131072;
 constexpr uint32_t kTailLanes = 256u * 4u * 3u * 64u;
 
