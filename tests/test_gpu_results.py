@@ -95,7 +95,8 @@ def test_result_memory_is_the_callers(torch_cuda, width, height):
 @pytest.mark.parametrize("width,height", [(418, 418), (419, 418), (836, 418), (1277, 719)])
 def test_whole_frames_from_several_threads(torch_cuda, width, height):
     """Frames just below and above the size read in pieces, of one piece and
-    of several with a remainder, into ordinary and page-locked memory."""
+    of several with a remainder, into ordinary memory, at odd addresses too,
+    and into page-locked memory."""
     r = renderer(width, height, spp=1)
     r.render_samples(0, 1)
     want = r.render_task(wpt.Task(0, 0, 0, 1, 0, 0, width, height))
@@ -115,3 +116,8 @@ def test_whole_frames_from_several_threads(torch_cuda, width, height):
     locked = np.ctypeslib.as_array(C.cast(block, C.POINTER(C.c_float)), want.shape).copy()
     wpt.check(lib.wpt_host_free(block), "wpt_host_free")
     assert all(np.array_equal(g, want) for g in got + [locked])
+    for shift in (1, 2, 3):
+        odd = np.full(want.size + 8, -1.0, np.float32)
+        wpt.check(lib.wpt_renderer_read_framebuffer(r._h, odd[shift:].ctypes.data, None), "wpt_renderer_read_framebuffer")
+        assert np.array_equal(odd[shift:shift + want.size], want.ravel())
+        assert np.all(odd[:shift] == -1.0) and np.all(odd[shift + want.size:] == -1.0)

@@ -81,13 +81,32 @@ struct DeviceArena {
     }
 };
 
+// memcpy past the caches, for results larger than they are: 16 B stores that
+// do not read the lines they fill.
+void streamCopy(char* dst, const char* src, size_t n) {
+    typedef float Lane __attribute__((ext_vector_type(4)));
+    const size_t head = std::min(n, (16 - (reinterpret_cast<uintptr_t>(dst) & 15)) & 15);
+    std::memcpy(dst, src, head);
+    dst += head;
+    src += head;
+    n -= head;
+    for (; n >= 64; n -= 64, dst += 64, src += 64) {
+        Lane v[4];
+        std::memcpy(v, src, sizeof v);
+        for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(v[k], reinterpret_cast<Lane*>(dst) + k);
+    }
+    std::memcpy(dst, src, n);
+    __atomic_thread_fence(__ATOMIC_SEQ_CST);  // such stores are not ordered by themselves
+}
+
 // Device results on their way into ordinary host memory: through two
 // page-locked halves of fixed size, the link filling one while the CPU empties
 // the other.  A 1080p framebuffer (25 MB) into memory that is already mapped
-// takes 990 us so, 1380 us by one hipMemcpy, whose staging takes turns with its
-// transfers (into page-locked memory, 470 us; halves of 1 to 4 MiB alike).  One
-// hipMemcpy2D of a 97x61 tile into ordinary memory makes its task 664 us, where
-// rows that land in page-locked memory make it 313.
+// takes 760 us so (980 us emptied by memcpy), 1380 us by one hipMemcpy, whose
+// staging takes turns with its transfers (into page-locked memory, 470 us;
+// halves of 1 to 4 MiB alike).  One hipMemcpy2D of a 97x61 tile into ordinary
+// memory makes its task 664 us, where rows that land in page-locked memory make
+// it 313.
 class ReadBack {
     static constexpr size_t kHalf = size_t(1) << 21;
     std::mutex mutex;  // reads of one owner may come from several threads
@@ -1230,7 +1249,7 @@ WPT_API int wpt_renderer_read_framebuffer(wpt_renderer* r, float* host, uint32_t
     size_t n = 3 * static_cast<size_t>(r->config.width) * r->config.height;
     if (ReadBack::worthwhile(sizeof(float) * n) && !knownToHip(host) && r->readBack.ready()) {
         auto take = [&](size_t at, const char* data, size_t count) {
-            std::memcpy(reinterpret_cast<char*>(host) + at, data, count);
+            streamCopy(reinterpret_cast<char*>(host) + at, data, count);
         };
         hipError_t e = r->readBack.copy(r->ctx.framebuffer, sizeof(float) * n, r->stream, take);
         if (e != hipSuccess) return hipFail(e, "framebuffer read-back");
