@@ -178,12 +178,10 @@ WPT_HD bool slab(const RayInv& r, float mnx, float mny, float mnz, float mxx, fl
 // passes some boxes more, so a candidate found in a leaf counts only if slab()
 // passes the leaf's own box (leafOpen; slotOpen for TLAS leaves and for the
 // clipped triangles of spatial splits): slab's distances grow with the box, so
-// that this one test stands for the boxes around it, and the candidates are
-// those of a walk that tests every box with slab().  Which of two counts can
-// still depend on the order of visits, where a triangle is hit a little before
-// the ray enters its box (rounding at an edge) and the other's distance lies
-// between: of rays aimed at edges 1 in 1e5 (overlapping boxes of a median tree)
-// to about 1 in 1e7 (SAH) hit the neighbour that a binary walk does not.
+// that this one test stands for the boxes around it, and hits are those of a
+// binary walk that tests every box with slab() in the same order (visitQuad;
+// the biases can put two entries in another order when origin * inv is a
+// million times their distances: 1 of 100 million rays aimed at edges).
 // Rays with a component outside 2^-60 .. 2^60 in size (a zero component of the
 // direction has an infinite inverse), which would overflow, take slab() at
 // every node: their nearBias.x is NaN.
@@ -285,8 +283,9 @@ WPT_HD bool popLive(Stack& stack, uint32_t base, float reach, uint32_t& cur) {
     return false;
 }
 
+// As a binary walk: the right one first unless the left one is nearer.
 WPT_HD void orderPair(float& ta, uint32_t& a, float& tb, uint32_t& b) {
-    bool swap = tb < ta;
+    bool swap = tb <= ta;
     float t = swap ? tb : ta;
     uint32_t c = swap ? b : a;
     tb = swap ? ta : tb;
@@ -295,27 +294,47 @@ WPT_HD void orderPair(float& ta, uint32_t& a, float& tb, uint32_t& b) {
     a = c;
 }
 
-// visitQuad for the rays that are not regular().
-WPT_HD void exactBoxes(const QuadNode& n, const RayInv& r, float closestT, float t[kQuadChildren]) {
+// visitQuad for the rays that are not regular(): the children's entry distances
+// and those of the two pairs' unions.
+WPT_HD void exactBoxes(const QuadNode& n, const RayInv& r, float closestT, float t[kQuadChildren], float pair[2]) {
     for (uint32_t k = 0; k < kQuadChildren; ++k) {
         float tmin;
         bool hit = n.child[k] != kInvalid &&
             slab(r, n.mn[0][k], n.mn[1][k], n.mn[2][k], n.mx[0][k], n.mx[1][k], n.mx[2][k], closestT, tmin);
         t[k] = hit ? tmin : kBoxMissed;
     }
+    for (uint32_t k = 0; k < 2; ++k) {
+        float mn[3], mx[3];
+        for (int c = 0; c < 3; ++c) {
+            mn[c] = fminf(n.mn[c][2 * k], n.mn[c][2 * k + 1]);
+            mx[c] = fmaxf(n.mx[c][2 * k], n.mx[c][2 * k + 1]);
+        }
+        (void)slab(r, mn[0], mn[1], mn[2], mx[0], mx[1], mx[2], closestT, pair[k]);
+    }
 }
 
-// One interior node: the nearest child whose box the ray reaches becomes
-// `cur`, the others are pushed, the farthest first; false when there is none.
+// One interior node: the first child whose box the ray reaches becomes `cur`,
+// the others are pushed, the last first; false when there is none.
 // A walk is bound by VALU issue where the chip is full and by the latency of
 // its chain of node fetches where it is not.  Four boxes a visit halve the
-// chain, for the 128 B line that is fetched either way, and take about 100
+// chain, for the 128 B line that is fetched either way, and take about 110
 // vector instructions where two binary visits with ordered planes took 150:
-// sphere field 1920x1080, 64 spp, closest-hit passes 58.4 -> 39.7 ms; terrain,
-// 16 spp, 66 -> 49 ms and event rays 62 -> 46 ms; 2M camera rays 529 -> 342 us.
+// sphere field 1920x1080, 64 spp, closest-hit passes 58.4 -> 39.9 ms; terrain,
+// 16 spp, 66 -> 49 ms and event rays 62 -> 45 ms; 2M camera rays 529 -> 338 us.
 // Which plane of an axis a ray enters through depends on the sign of its
 // direction alone, so a lane loads each node's entry and exit planes as such
 // (minima at byte 0, 16, 32, maxima 48 further) instead of ordering them.
+// The order is that of a binary walk: the pair whose union is entered first,
+// its nearer child first, distances behind the origin included.  Which of two
+// triangles counts depends on it where one is hit a little before the ray
+// enters its box (rounding at an edge) and the other's distance lies between:
+// with all four children ordered by their own clamped distances up to 10 of
+// 400,000 rays aimed at edges under a median tree hit another triangle than in a
+// binary walk, so none.  That order took 2 to 5% less time (a child of a child
+// could fill a slot left free, and fewer registers were live; with the entries
+// of all four children computed first, 3 to 5 spills less but terrain 139.9 ->
+// 146.2 ms; with one slack for the three axes instead of biases, flat trees 350
+// -> 785 us, as rays almost parallel to an axis pass nearly every box).
 template <class Stack>
 WPT_HD bool visitQuad(const QuadNode* nodes, const BoxRay& r, float closestT, uint32_t& cur, Stack& stack) {
     const char* p = reinterpret_cast<const char*>(nodes + cur);
@@ -325,31 +344,49 @@ WPT_HD bool visitQuad(const QuadNode* nodes, const BoxRay& r, float closestT, ui
                  ny = *reinterpret_cast<const float4*>(p + oy + 16), fy = *reinterpret_cast<const float4*>(p + (oy ^ 48u) + 16),
                  nz = *reinterpret_cast<const float4*>(p + oz + 32), fz = *reinterpret_cast<const float4*>(p + (oz ^ 48u) + 32);
     const uint4 child = *reinterpret_cast<const uint4*>(p + 96);
-    auto box = [&](float nx, float ny, float nz, float fx, float fy, float fz) {
-        float tmin = fmaxf(fmaxf(fmaxf(fmaf(nx, r.inv.x, r.nearBias.x), fmaf(ny, r.inv.y, r.nearBias.y)),
-                               fmaf(nz, r.inv.z, r.nearBias.z)), kRayMinDistance);
+    auto enter = [&](float nx, float ny, float nz) {
+        return Vec3(fmaf(nx, r.inv.x, r.nearBias.x), fmaf(ny, r.inv.y, r.nearBias.y), fmaf(nz, r.inv.z, r.nearBias.z));
+    };
+    auto box = [&](const Vec3& e, float fx, float fy, float fz) {
+        float tmin = fmaxf(fmaxf(e.x, e.y), e.z);
         float tmax = fminf(fminf(fminf(fmaf(fx, r.inv.x, r.farBias.x), fmaf(fy, r.inv.y, r.farBias.y)),
                                fmaf(fz, r.inv.z, r.farBias.z)), closestT);
-        return tmin <= boxReach(tmax) ? tmin : kBoxMissed;
+        return fmaxf(tmin, kRayMinDistance) <= boxReach(tmax) ? tmin : kBoxMissed;
     };
-    float t0 = box(nx.x, ny.x, nz.x, fx.x, fy.x, fz.x);
-    float t1 = box(nx.y, ny.y, nz.y, fx.y, fy.y, fz.y);
-    float t2 = box(nx.z, ny.z, nz.z, fx.z, fy.z, fz.z);
-    float t3 = box(nx.w, ny.w, nz.w, fx.w, fy.w, fz.w);
+    auto both = [](const Vec3& a, const Vec3& b) {
+        return fmaxf(fmaxf(fminf(a.x, b.x), fminf(a.y, b.y)), fminf(a.z, b.z));
+    };
+    const Vec3 e0 = enter(nx.x, ny.x, nz.x), e1 = enter(nx.y, ny.y, nz.y);
+    float t0 = box(e0, fx.x, fy.x, fz.x), t1 = box(e1, fx.y, fy.y, fz.y), left = both(e0, e1);
+    const Vec3 e2 = enter(nx.z, ny.z, nz.z), e3 = enter(nx.w, ny.w, nz.w);
+    float t2 = box(e2, fx.z, fy.z, fz.z), t3 = box(e3, fx.w, fy.w, fz.w), right = both(e2, e3);
     if (!r.regular()) {
-        float t[kQuadChildren];
-        exactBoxes(nodes[cur], r.exact(), closestT, t);
+        float t[kQuadChildren], pair[2];
+        exactBoxes(nodes[cur], r.exact(), closestT, t, pair);
         t0 = t[0];
         t1 = t[1];
         t2 = t[2];
         t3 = t[3];
+        left = pair[0];
+        right = pair[1];
     }
     uint32_t c0 = child.x, c1 = child.y, c2 = child.z, c3 = child.w;
     orderPair(t0, c0, t1, c1);
     orderPair(t2, c2, t3, c3);
-    orderPair(t0, c0, t2, c2);
-    orderPair(t1, c1, t3, c3);
-    orderPair(t1, c1, t2, c2);
+    if (t2 < kBoxMissed && (t0 == kBoxMissed || right <= left)) {
+        float t = t0;
+        t0 = t2;
+        t2 = t;
+        t = t1;
+        t1 = t3;
+        t3 = t;
+        uint32_t c = c0;
+        c0 = c2;
+        c2 = c;
+        c = c1;
+        c1 = c3;
+        c3 = c;
+    }
     if (t3 < kBoxMissed) stack.push(c3, t3);
     if (t2 < kBoxMissed) stack.push(c2, t2);
     if (t1 < kBoxMissed) stack.push(c1, t1);

@@ -42,9 +42,8 @@ struct alignas(16) BvhNode {
 static_assert(sizeof(BvhNode) == 64, "BvhNode must be one 64 B chunk");
 
 // Four-wide node, the form the kernels walk: node i holds binary node i's
-// grandchildren (a child that is a leaf stays, and then the largest
-// grandchild is opened once more), in the binary tree's node and slot
-// numbers, so each is made from the binary tree by itself; the nodes that
+// grandchildren (a child that is a leaf stays), in the binary tree's node and
+// slot numbers, so each is made from the binary tree by itself; the nodes that
 // others opened are never reached.  Planes of the four children side by side,
 // 16 B per plane; an unused child (kInvalid) has an empty box.
 constexpr uint32_t kQuadChildren = 4;
@@ -56,60 +55,35 @@ struct alignas(128) QuadNode {
 };
 static_assert(sizeof(QuadNode) == 128, "QuadNode must be one 128 B line");
 
-// Quad node i from binary node i: its two children, each opened into its own
-// two if it is interior, then the largest interior child opened until there
-// are four.
+// Quad node i from binary node i: slots 0 and 1 its left child's two, 2 and 3
+// its right child's; a child that is a leaf takes the first slot of its pair.
 WPT_HD QuadNode quadNode(const BvhNode* nodes, uint32_t i) {
-    float box[kQuadChildren][6];
-    uint32_t child[kQuadChildren];
-    auto open = [&](uint32_t node, uint32_t left, uint32_t right) {
-        const BvhNode n = nodes[node];
-        const float l[6] = {n.lminx, n.lminy, n.lminz, n.lmaxx, n.lmaxy, n.lmaxz};
-        const float r[6] = {n.rminx, n.rminy, n.rminz, n.rmaxx, n.rmaxy, n.rmaxz};
-        for (int k = 0; k < 6; ++k) {
-            box[left][k] = l[k];
-            box[right][k] = r[k];
-        }
-        child[left] = n.left;
-        child[right] = n.right;
-    };
-    open(i, 0u, 1u);
-    uint32_t used = 2u;
-    const bool openLeft = !(child[0] & kLeafBit), openRight = !(child[1] & kLeafBit);
-    if (openLeft) open(child[0], 0u, used++);
-    if (openRight) open(child[1], 1u, used++);
-    while (used < kQuadChildren) {
-        uint32_t best = kInvalid;
-        float area = -1.0f;
-        for (uint32_t k = 0; k < used; ++k) {
-            if (child[k] & kLeafBit) continue;
-            float dx = box[k][3] - box[k][0], dy = box[k][4] - box[k][1], dz = box[k][5] - box[k][2];
-            float a = dx * dy + dy * dz + dz * dx;
-            if (best == kInvalid || a > area) {
-                best = k;
-                area = a;
-            }
-        }
-        if (best == kInvalid) break;
-        open(child[best], best, used++);
-    }
-    const float inf = __builtin_inff();
-    for (uint32_t k = used; k < kQuadChildren; ++k) {
-        child[k] = kInvalid;
-        for (int c = 0; c < 3; ++c) {
-            box[k][c] = inf;
-            box[k][3 + c] = -inf;
-        }
-    }
     QuadNode q;
-    for (uint32_t k = 0; k < kQuadChildren; ++k) {
-        for (int c = 0; c < 3; ++c) {
-            q.mn[c][k] = box[k][c];
-            q.mx[c][k] = box[k][3 + c];
-        }
-        q.child[k] = child[k];
+    auto set = [&](uint32_t k, uint32_t child, float mnx, float mny, float mnz, float mxx, float mxy, float mxz) {
+        q.child[k] = child;
         q.pad[k] = 0u;
-    }
+        q.mn[0][k] = mnx;
+        q.mn[1][k] = mny;
+        q.mn[2][k] = mnz;
+        q.mx[0][k] = mxx;
+        q.mx[1][k] = mxy;
+        q.mx[2][k] = mxz;
+    };
+    auto open = [&](const BvhNode& n, uint32_t left, uint32_t right) {
+        set(left, n.left, n.lminx, n.lminy, n.lminz, n.lmaxx, n.lmaxy, n.lmaxz);
+        set(right, n.right, n.rminx, n.rminy, n.rminz, n.rmaxx, n.rmaxy, n.rmaxz);
+    };
+    const float inf = __builtin_inff();
+    const BvhNode n = nodes[i];
+    open(n, 0u, 2u);
+    if (n.left & kLeafBit)
+        set(1u, kInvalid, inf, inf, inf, -inf, -inf, -inf);
+    else
+        open(nodes[n.left], 0u, 1u);
+    if (n.right & kLeafBit)
+        set(3u, kInvalid, inf, inf, inf, -inf, -inf, -inf);
+    else
+        open(nodes[n.right], 2u, 3u);
     return q;
 }
 
