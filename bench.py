@@ -62,15 +62,15 @@ RAY_IN_B, HIT_OUT_B = 24, 28
 # (profiles/pmc_kTrace_sphere_field_1080p_64spp.md).  kBatch: one 64-sample
 # frame of the regenerating scheduler
 # (profiles/pmc_kBatch_sphere_field_1080p_64spp.md).
-MEASURED_TRAFFIC = {("kTrace", 64): 35.07e9 / 12, ("kBatch", 64): 29.83e9}
+MEASURED_TRAFFIC = {("kTrace", 64): 36.31e9 / 12, ("kBatch", 64): 29.95e9}
 MEASURED_COUNTERS = {
-    ("kTrace", 64): {"l2_hit": 0.477, "valu_busy": 0.956, "waves_per_cu": 12.12, "wait_any": 0.464,
-                     "lanes_active": 0.331, "l1_hit": 0.921, "ta_busy": 0.522, "l1_to_l2_latency_cycles": 322},
-    ("kBatch", 64): {"l2_hit": 0.596, "valu_busy": 0.459, "waves_per_cu": 8.89, "wait_any": 0.635,
-                     "lanes_active": 0.213},
+    ("kTrace", 64): {"l2_hit": 0.478, "valu_busy": 0.965, "waves_per_cu": 12.17, "wait_any": 0.450,
+                     "lanes_active": 0.328, "l1_hit": 0.921, "ta_busy": 0.516, "l1_to_l2_latency_cycles": 322},
+    ("kBatch", 64): {"l2_hit": 0.631, "valu_busy": 0.444, "waves_per_cu": 8.66, "wait_any": 0.631,
+                     "lanes_active": 0.210},
 }
 LIMITERS = {
-    "kTrace": "VALU issue: busy 96% of the time with a third of the lanes active (turns of one visit kind per wave); "
+    "kTrace": "VALU issue: busy 97% of the time with a third of the lanes active (turns of one visit kind per wave); "
               "HBM carries a ninth of its peak",
     "kBatch": "chains of dependent node fetches at 3 waves per SIMD, with a fifth of the lanes of a VALU instruction "
               "active where shading and shadow rays take turns",
