@@ -181,7 +181,9 @@ WPT_HD bool slab(const RayInv& r, float mnx, float mny, float mnz, float mxx, fl
 // that this one test stands for the boxes around it, and hits are those of a
 // binary walk that tests every box with slab() in the same order (visitQuad;
 // the biases can put two entries in another order when origin * inv is a
-// million times their distances: 1 of 150 million rays aimed at edges).
+// million times their distances: 1 of 150 million rays aimed at edges; clipped
+// boxes reach out of those around them by rounding, where a binary walk misses a
+// few hits at their seams that this one finds: 1 in 100,000 such rays).
 // Rays with a component outside 2^-60 .. 2^60 in size (a zero component of the
 // direction has an infinite inverse), which would overflow, take slab() at
 // every node: their nearBias.x is NaN.
